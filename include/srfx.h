@@ -61,7 +61,12 @@ enum srfx_status {
  * flag one lane per event, except the projection of a plan's OSEM step
  * (srfx_tor_plan_osem_subset), which takes four.
  * Threads per block: SRFX_BLOCK_256 (default), SRFX_BLOCK_64, SRFX_BLOCK_128.
- * Results agree to FP32 rounding across schedules. */
+ * Results agree to FP32 rounding across schedules.
+ * Without any schedule flag a large scatter (backprojection, adjoint, Maplors,
+ * OSEM pass; ~2.4e6 weights and up) runs binned: its events are listed by image
+ * tile on the device and every tile accumulated in LDS, with a stream-ordered
+ * workspace of up to 256 MiB from the device's memory pool (a stream under
+ * capture, or a failed allocation, keeps the kernels without workspace). */
 #define SRFX_LPE_SHIFT 4
 #define SRFX_LPE_1 (1u << SRFX_LPE_SHIFT)
 #define SRFX_LPE_4 (2u << SRFX_LPE_SHIFT)

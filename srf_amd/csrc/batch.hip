@@ -43,8 +43,7 @@ struct EvChunk {
 };
 
 // Box classes of the batch's jobs: 0 = candidate box 3 with every event on
-// the 3 x 2 box and a y-fastest flush (the single-walk scatter), 1 = other
-// box-3 jobs, 2 = box 4, 3 = chord walk.  Each class has its own work lists
+// the 3 x 2 box (the single-walk scatter), 1 = other box-3 jobs, 2 = box 4, 3 = chord walk.  Each class has its own work lists
 // and persistent kernels, so that a kernel holds only its class's walk (and
 // its registers).
 constexpr int kBoxClasses = 4;
@@ -52,7 +51,7 @@ constexpr int kBoxClasses = 4;
 inline int box_class(const TorParams &p, bool single_walk)
 {
     if (p.box == 3)
-        return single_walk && flush_y_fastest(p) ? 0 : 1;
+        return single_walk ? 0 : 1;
     return p.box == 4 ? 2 : 3;
 }
 
@@ -107,18 +106,6 @@ __global__ __launch_bounds__(256) void batch_update(const VoxRange *__restrict__
         long long j = i - r[k].off;
         r[k].x[j] = (r[k].x[j] * r[k].e[j]) * r[k].bp[j];
     }
-}
-
-// Next work item of a persistent block (the same value in every thread).
-__device__ __forceinline__ int next_item(unsigned *counter)
-{
-    __shared__ int item;
-    if (threadIdx.x == 0)
-        item = (int)atomicAdd(counter, 1u);
-    __syncthreads();
-    const int c = __builtin_amdgcn_readfirstlane(item);
-    __syncthreads();
-    return c;
 }
 
 // Next work item of a persistent wave (the same value in every lane; every
@@ -180,12 +167,7 @@ __global__ __launch_bounds__(256, ONE ? 5 : (NB == 4 ? 3 : 4)) void batch_scatte
         const TileWork w = work[c];
         const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(w.job)];
         const TileChunk ch{w.tile, w.start, w.count, 0};
-        if constexpr (ONE)
-            scatter_chunk<kBack, NB, true, true, true>(job.p, job.g, ch, job.list, job.rec, ldsd);
-        else if (flush_y_fastest(job.p))
-            scatter_chunk<kBack, NB, true, true>(job.p, job.g, ch, job.list, job.rec, ldsd);
-        else
-            scatter_chunk<kBack, NB, true, false>(job.p, job.g, ch, job.list, job.rec, ldsd);
+        scatter_chunk<kBack, NB, true, ONE>(job.p, job.g, ch, job.list, job.rec, ldsd);
     }
 }
 

@@ -62,7 +62,6 @@ unsigned lds_bytes_scatter(const TileGeom &g)
 
 // Largest tile count whose per-workgroup counters (3 per tile) fit in 64 KB.
 constexpr int kLdsTiles = 16384 / 3;
-constexpr unsigned kLdsPerCU = 160u * 1024u; // LDS of one CU
 
 template <bool FILL>
 void launch_pass(const TorParams &p, const TileGeom &g, const PlanArgs &a, hipStream_t st)
@@ -384,16 +383,7 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
         a.ntiles = l.nt;
         a.nplans = ps.K;
         a.lds = 3u * sizeof(int) * l.nt <= 65536u;
-        // the longest listing queues that keep three workgroups of the fill
-        // pass per CU (with fewer, at C5's 2816 tiles, queues of 959 entries
-        // in 64 KB: 115 ms against 101 ms without queues)
-        a.queue = 0;
-        const unsigned qbudget = kLdsPerCU / 3u;
-        if (l.nt < (1 << 24) &&
-            fill_queue_lds(kFillQueueMin) + 3u * sizeof(int) * l.nt <= qbudget)
-            a.queue = std::min<int>(kFillQueue, (int)((qbudget - 3u * sizeof(int) * l.nt -
-                                                       fill_queue_lds(0)) /
-                                                      (4u * sizeof(int))));
+        a.queue = fill_queue_entries(l.nt);
         a.first = (const int64_t *)(tmp + l.head);
         a.rec = (float4 *const *)(tmp + l.head + sizeof(int64_t) * (ps.K + 1));
         a.list = (int *const *)(tmp + l.head + sizeof(int64_t) * (ps.K + 1) +
@@ -600,54 +590,35 @@ int plan_build_set(srfx_tor_plan_s *const *pls, int K, const int64_t *first, con
     return plan_build_sets({PlanSet{pls, K, first, lors, chunk}}, st);
 }
 
-template <int MODE, bool VREC, bool YF>
-void launch_scatter_l(const TorParams &p, const srfx_tor_plan_s *pl, dim3 grid, dim3 block,
-                      unsigned sh, hipStream_t st)
+template <int MODE, bool VREC>
+void launch_scatter(const TorParams &p, const srfx_tor_plan_s *pl, dim3 grid, dim3 block,
+                    unsigned sh, hipStream_t st)
 {
     switch (p.box) {
     case 3:
         // plans whose events all walk the 3 x 2 box, with tiles that let five
         // workgroups share a CU's LDS: the single-walk kernel
-        if constexpr (YF) {
-            if (pl->one && 5u * sh <= kLdsPerCU) {
-                hipLaunchKernelGGL((tile_scatter<MODE, 3, VREC, true, true>), grid, block, sh, st,
-                                   p, pl->g, pl->chunks, pl->list, pl->rec);
-                break;
-            }
-        }
-        hipLaunchKernelGGL((tile_scatter<MODE, 3, VREC, YF>), grid, block, sh, st, p, pl->g,
-                           pl->chunks, pl->list, pl->rec);
+        if (pl->one && 5u * sh <= kCuLds)
+            hipLaunchKernelGGL((tile_scatter<MODE, 3, VREC, true>), grid, block, sh, st, p, pl->g,
+                               pl->chunks, pl->list, pl->rec);
+        else
+            hipLaunchKernelGGL((tile_scatter<MODE, 3, VREC>), grid, block, sh, st, p, pl->g,
+                               pl->chunks, pl->list, pl->rec);
         break;
     case 4:
         // the 4 x 3 box walk alone: four waves per SIMD instead of three
-        if constexpr (YF) {
-            if (pl->one && 4u * sh <= kLdsPerCU) {
-                hipLaunchKernelGGL((tile_scatter<MODE, 4, VREC, true, true>), grid, block, sh, st,
-                                   p, pl->g, pl->chunks, pl->list, pl->rec);
-                break;
-            }
-        }
-        hipLaunchKernelGGL((tile_scatter<MODE, 4, VREC, YF>), grid, block, sh, st, p, pl->g,
-                           pl->chunks, pl->list, pl->rec);
+        if (pl->one && 4u * sh <= kCuLds)
+            hipLaunchKernelGGL((tile_scatter<MODE, 4, VREC, true>), grid, block, sh, st, p, pl->g,
+                               pl->chunks, pl->list, pl->rec);
+        else
+            hipLaunchKernelGGL((tile_scatter<MODE, 4, VREC>), grid, block, sh, st, p, pl->g,
+                               pl->chunks, pl->list, pl->rec);
         break;
     default:
-        hipLaunchKernelGGL((tile_scatter<MODE, 0, VREC, YF>), grid, block, sh, st, p, pl->g,
+        hipLaunchKernelGGL((tile_scatter<MODE, 0, VREC>), grid, block, sh, st, p, pl->g,
                            pl->chunks, pl->list, pl->rec);
         break;
     }
-}
-
-// The LDS tile runs fastest along the output's smaller stride (op y for the
-// world layout of the axis groups, op x for a contiguous op frame), so the
-// flush's atomics are coalesced.
-template <int MODE, bool VREC>
-void launch_scatter(const TorParams &p, const srfx_tor_plan_s *pl, dim3 grid, dim3 block,
-                    unsigned sh, hipStream_t st)
-{
-    if (flush_y_fastest(p))
-        launch_scatter_l<MODE, VREC, true>(p, pl, grid, block, sh, st);
-    else
-        launch_scatter_l<MODE, VREC, false>(p, pl, grid, block, sh, st);
 }
 
 int plan_scatter(srfx_tor_plan_s *pl, int mode, const float *vals, float *image,

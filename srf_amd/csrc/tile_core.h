@@ -427,6 +427,21 @@ __host__ __device__ constexpr unsigned fill_queue_lds(int qcap)
     return 256u * sizeof(FillEvent) + 4u * (unsigned)qcap * sizeof(int) + 4u * sizeof(int);
 }
 
+constexpr unsigned kCuLds = 160u * 1024u; // LDS of one CU
+
+// Queue entries per wave of the fill pass over nt tiles (0: no queues): the
+// longest queues that keep three workgroups of the pass per CU (with fewer,
+// at 2816 tiles, queues of 959 entries in 64 KB: 115 ms against 101 ms
+// without queues for a 300M-event plan set).
+inline int fill_queue_entries(int nt)
+{
+    const unsigned budget = kCuLds / 3u, ctr = 3u * sizeof(int) * (unsigned)nt;
+    if (nt >= (1 << 24) || fill_queue_lds(kFillQueueMin) + ctr > budget)
+        return 0;
+    const int q = (int)((budget - ctr - fill_queue_lds(0)) / (4u * sizeof(int)));
+    return q < kFillQueue ? q : kFillQueue;
+}
+
 // listing_slices from a queued event's fields
 __device__ __forceinline__ void listing_slices(const TorParams &p, const TileBox &b,
                                                const FillEvent &f, int &s0, int &s1)
@@ -686,12 +701,9 @@ __device__ __forceinline__ float window_walk(const TorParams &p, const TileGeom 
     return acc;
 }
 
-// One listing: its slices s0..s1 inside the tile (listing_slices), each
-// through the NB x NB candidate box clipped to the window when the event's
-// box fits, else the clipped chord walk.
 // The scatter of one listing (slices s0..s1) through its BX x BY candidate box
-// into a y-fastest FP64 LDS tile: the box walk of slice_box<1, BX, BY, 2>
-// with less work per slice.
+// into a y-fastest FP64 LDS tile: the scatter of slice_box<1, BX, BY> with
+// less work per slice.
 //   * The box's clip to the patch [0, P) and the window as float bounds
 //     (lo, hi) on its first column / row, so the offsets need no integer
 //     round trip; clipped candidates get an infinite term (neither kept nor
@@ -795,42 +807,53 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     }
 }
 
-template <int KIND, int NB, bool YF, typename T>
-__device__ __forceinline__ float tile_event(const TorParams &p, const TileGeom &g,
-                                            const TileBox &b, const Event &ev, const Track &t,
-                                            bool tof, float scale, int s0, int s1, T *lds)
+// The scatter of one listing whose box is larger than the compiled one: the
+// clipped chord walk of each slice into the y-fastest tile.  The scale rides
+// in amp (one product per slice, not per voxel), with the TOF constant folded
+// into it once.
+__device__ __forceinline__ void scatter_chords(const TorParams &p, const TileGeom &g,
+                                               const TileBox &b, const Event &ev, const Track &t,
+                                               bool tof, float scale, int s0, int s1, double *lds)
+{
+    const float ts = p.tofk * scale;
+    for (int s = s0; s <= s1; s++) {
+        Cross c;
+        cross_at(p, ev, t, s, c);
+        const float amp = tof ? tof_exp(p, ev, t, s) * ts : scale;
+        window_walk<1, true>(p, g, b, ev, t, c, amp, s, scale, lds);
+    }
+}
+
+// The gather of one listing (slices s0..s1) from an x-fastest LDS tile:
+// returns its projection over the tile.
+template <int NB>
+__device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom &g,
+                                              const TileBox &b, const Event &ev, const Track &t,
+                                              bool tof, int s0, int s1, float *lds)
 {
     constexpr int NBB = NB > 1 ? NB : 2;
     const int shape = box_shape<NB>(t);
     const int P = p.patch;
-    const float ts = p.tofk * scale;
     float acc = 0.0f;
     for (int s = s0; s <= s1; s++) {
         Cross c;
         cross_at(p, ev, t, s, c);
-        // scatters: the scale rides in amp (one product per slice, not per
-        // voxel), with the TOF constant folded into it once
-        float amp = KIND == 1 ? (tof ? tof_exp(p, ev, t, s) * ts : scale)
-                              : (tof ? tof_factor(p, ev, t, s) : 1.0f);
+        const float amp = tof ? tof_factor(p, ev, t, s) : 1.0f;
         if (NB > 0 && shape) {
             PatchIdx idx;
-            idx.base = lds_index<YF>(g, b, s, c.ix0, c.iy0);
-            idx.si = YF ? g.Wy : 1;
-            idx.sj = YF ? 1 : g.Wx;
-            const float *src = nullptr;
-            if constexpr (KIND == 0)
-                src = lds;
+            idx.base = lds_index<false>(g, b, s, c.ix0, c.iy0);
+            idx.si = 1;
+            idx.sj = g.Wx;
             const int il = max(0, b.x0 - c.ix0), ih = min(P - 1, b.x1 - c.ix0);
             const int jl = max(0, b.y0 - c.iy0), jh = min(P - 1, b.y1 - c.iy0);
-            constexpr int L = YF ? 2 : 1;
             if (shape == 1)
-                acc += slice_box<KIND, NBB, NBB - 1, L>(p, ev, t, c, amp, s, scale, il, ih, jl,
-                                                        jh, idx, src, lds);
+                acc += slice_box<0, NBB, NBB - 1, true>(p, ev, t, c, amp, s, il, ih, jl, jh, idx,
+                                                        lds, lds);
             else
-                acc += slice_box<KIND, NBB, NBB, L>(p, ev, t, c, amp, s, scale, il, ih, jl, jh,
-                                                    idx, src, lds);
+                acc += slice_box<0, NBB, NBB, true>(p, ev, t, c, amp, s, il, ih, jl, jh, idx,
+                                                    lds, lds);
         } else {
-            acc += window_walk<KIND, YF>(p, g, b, ev, t, c, amp, s, scale, lds);
+            acc += window_walk<0, false>(p, g, b, ev, t, c, amp, s, 0.0f, lds);
         }
     }
     return acc;
@@ -903,14 +926,67 @@ __global__ __launch_bounds__(256, NB == 3 && FRAME && LPE <= 4 ? 5 : 4) void rec
 }
 
 
+// Flush of a y-fastest LDS tile (voxel (s, x, y) at (s Wx + x) Wy + y) into
+// p.out with one FP32 atomic per non-zero voxel, consecutive lanes along the
+// output's smaller in-slice stride: op y (YF, the world layout of the axis
+// groups) or op x (a contiguous op frame).  Tile element (c, m, f), f along
+// that axis, m the other one and c the slice, advances by the block size each
+// step: indices, LDS element and output offset with carries instead of
+// divisions by the tile extents.
+template <bool YF>
+__device__ __forceinline__ void flush_tile(const TorParams &p, const TileGeom &g,
+                                           const TileBox &b, const double *ldsd)
+{
+    const int nv = g.S * g.Wy * g.Wx;
+    const int na = YF ? g.Wy : g.Wx, nb = YF ? g.Wx : g.Wy;
+    const int oa = YF ? p.oy : p.ox, ob = YF ? p.ox : p.oy;
+    const int la = YF ? b.y1 - b.y0 : b.x1 - b.x0, lb = YF ? b.x1 - b.x0 : b.y1 - b.y0;
+    const int lc = b.sb - b.sa;
+    int f = threadIdx.x % na, m, c;
+    {
+        const int r = threadIdx.x / na;
+        m = r % nb;
+        c = r / nb;
+    }
+    const int df = blockDim.x % na, dr = blockDim.x / na;
+    const int dm = dr % nb, dc = dr / nb;
+    float *const base = p.out + ((int64_t)b.x0 * p.ox + (int64_t)b.y0 * p.oy + (int64_t)b.sa * p.oz);
+    int off = f * oa + m * ob + c * p.oz;
+    const int step = df * oa + dm * ob + dc * p.oz;
+    const int wrap_f = ob - na * oa, wrap_m = p.oz - nb * ob;
+    // LDS element: i itself for YF, else f Wy + m + c Wx Wy
+    const int ns = g.Wx * g.Wy;
+    int l = f * g.Wy + m + c * ns;
+    const int lstep = df * g.Wy + dm + dc * ns;
+    for (int i = threadIdx.x; i < nv; i += blockDim.x) {
+        const float v = (float)ldsd[YF ? i : l];
+        if (v != 0.0f && f <= la && m <= lb && c <= lc)
+            unsafeAtomicAdd(base + off, v);
+        f += df;
+        off += step;
+        l += lstep;
+        const bool cf = f >= na;
+        f -= cf ? na : 0;
+        off += cf ? wrap_f : 0;
+        l += cf ? 1 - ns : 0;
+        m += dm + (cf ? 1 : 0);
+        const bool cm = m >= nb;
+        m -= cm ? nb : 0;
+        off += cm ? wrap_m : 0;
+        l += cm ? ns - nb : 0;
+        c += dc + (cm ? 1 : 0);
+    }
+}
+
 // Scatter of one chunk (modes kBack, kMap, kAdj) into p.out, through the
-// FP64 LDS tile ldsd (S * Wy * Wx doubles).  Every thread of the workgroup
-// calls it; it synchronises the workgroup before and after the flush.
+// y-fastest FP64 LDS tile ldsd (S * Wy * Wx doubles).  Every thread of the
+// workgroup calls it; it synchronises the workgroup before and after the
+// flush.
 // VREC (kBack only): the backprojection scales 1/p that the record projection
 // stored in the event records (the OSEM step of a plan), not p.val.
 // ONE: every listing's event walks the NB x (NB - 1) box (a plan whose
 // events all have box shape 1); the other walks are left out of the kernel.
-template <int MODE, int NB, bool VREC = false, bool YF = false, bool ONE = false>
+template <int MODE, int NB, bool VREC = false, bool ONE = false>
 __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom &g,
                                               const TileChunk &ch,
                                               const int *__restrict__ list,
@@ -963,52 +1039,33 @@ __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom
             constexpr int NBB = NB > 1 ? NB : 2;
             constexpr bool POS = MODE == kBack; // scale 1/v with v > 1e-7
             const int shape = box_shape<NB>(t);
-            static_assert(!ONE || (YF && NB > 0), "the single walk is the y-fastest box walk");
-            if (ONE || (YF && NB > 0 && shape == 1))
+            static_assert(!ONE || NB > 0, "the single walk is a box walk");
+            if (ONE || (NB > 0 && shape == 1))
                 scatter_box_yf<NBB, NBB - 1, POS>(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
-            else if (YF && NB > 0 && shape == 2)
+            else if (NB > 0 && shape == 2)
                 scatter_box_yf<NBB, NBB, POS>(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
             else
-                tile_event<1, NB, YF>(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
+                scatter_chords(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
         }
     }
     __syncthreads();
-    // Flush.  Tile element i = (c * nb + m) * na + f (f along the fastest
-    // axis: y for YF, else x; m the middle one; c the slice) and its output
-    // offset advance by the block size each step, with carries instead of
-    // divisions by the tile extents.
-    const int na = YF ? g.Wy : g.Wx, nb = YF ? g.Wx : g.Wy;
-    const int oa = YF ? p.oy : p.ox, ob = YF ? p.ox : p.oy;
-    const int la = YF ? b.y1 - b.y0 : b.x1 - b.x0, lb = YF ? b.x1 - b.x0 : b.y1 - b.y0;
-    const int lc = b.sb - b.sa;
-    int f = threadIdx.x % na, m, c;
-    {
-        const int r = threadIdx.x / na;
-        m = r % nb;
-        c = r / nb;
-    }
-    const int df = blockDim.x % na, dr = blockDim.x / na;
-    const int dm = dr % nb, dc = dr / nb;
-    float *const base = p.out + ((int64_t)b.x0 * p.ox + (int64_t)b.y0 * p.oy + (int64_t)b.sa * p.oz);
-    int off = f * oa + m * ob + c * p.oz;
-    const int step = df * oa + dm * ob + dc * p.oz;
-    const int wrap_f = ob - na * oa, wrap_m = p.oz - nb * ob;
-    for (int i = threadIdx.x; i < nv; i += blockDim.x) {
-        const float v = (float)ldsd[i];
-        if (v != 0.0f && f <= la && m <= lb && c <= lc)
-            unsafeAtomicAdd(base + off, v);
-        f += df;
-        off += step;
-        const bool cf = f >= na;
-        f -= cf ? na : 0;
-        off += cf ? wrap_f : 0;
-        m += dm + (cf ? 1 : 0);
-        const bool cm = m >= nb;
-        m -= cm ? nb : 0;
-        off += cm ? wrap_m : 0;
-        c += dc + (cm ? 1 : 0);
-    }
+    if (flush_y_fastest(p))
+        flush_tile<true>(p, g, b, ldsd);
+    else
+        flush_tile<false>(p, g, b, ldsd);
     __syncthreads();
+}
+
+// Next work item of a persistent block (the same value in every thread).
+__device__ __forceinline__ int next_item(unsigned *counter)
+{
+    __shared__ int item;
+    if (threadIdx.x == 0)
+        item = (int)atomicAdd(counter, 1u);
+    __syncthreads();
+    const int c = __builtin_amdgcn_readfirstlane(item);
+    __syncthreads();
+    return c;
 }
 
 // The lanes of the wave whose v (0 <= v < 64) equals this lane's: one ballot
@@ -1160,13 +1217,13 @@ __global__ __launch_bounds__(256) void sort_chunks_many(const SortJob *__restric
 // NB x (NB - 1) box walk, NB = 3): five waves per SIMD in 96 VGPRs, for
 // tiles of at most a fifth of a CU's LDS (0.39 against 0.42 ms per 1M
 // events).
-template <int MODE, int NB, bool VREC, bool YF, bool ONE = false>
+template <int MODE, int NB, bool VREC, bool ONE = false>
 __global__ __launch_bounds__(256, NB == 4 ? (ONE ? 4 : 3) : (ONE ? 5 : 4)) void tile_scatter(
     TorParams p, TileGeom g, const TileChunk *__restrict__ chunks, const int *__restrict__ list,
     const float4 *__restrict__ rec)
 {
     extern __shared__ double ldsd[];
-    scatter_chunk<MODE, NB, VREC, YF, ONE>(p, g, chunks[blockIdx.x], list, rec, ldsd);
+    scatter_chunk<MODE, NB, VREC, ONE>(p, g, chunks[blockIdx.x], list, rec, ldsd);
 }
 
 // Gather of one chunk: partial[slot] = the listing's projection over the tile.
@@ -1200,8 +1257,7 @@ __global__ __launch_bounds__(256) void tile_gather(TorParams p, TileGeom g,
         unpack_walk(p, rec, e, ev, t);
         int s0, s1;
         listing_slices(p, b, ev, t, s0, s1);
-        const float acc = tile_event<0, NB, false>(p, g, b, ev, t, tof, 0.0f, s0, s1, lds);
-        partial[ch.start + j] = acc;
+        partial[ch.start + j] = gather_event<NB>(p, g, b, ev, t, tof, s0, s1, lds);
     }
 }
 

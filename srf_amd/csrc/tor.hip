@@ -2,6 +2,7 @@
 // The device code is in tor_core.h.
 #include <mutex>
 
+#include "binned.h"
 #include "tor_core.h"
 
 using namespace srfx;
@@ -60,6 +61,12 @@ static int tor_scatter_common(int mode, const float *lors, int64_t n, int64_t ld
     p.full_patch = (flags & SRFX_FULL_PATCH) ? 1 : 0;
     p.val = vals;
     p.out = image;
+    if (binned_ok(p, flags, st)) {
+        bool done = false;
+        rc = binned_scatter(mode, p, st, &done);
+        if (rc || done)
+            return rc;
+    }
     int nslab, inter;
     if (slab_schedule(flags, nslab, inter)) {
         switch (mode) {
@@ -152,6 +159,12 @@ extern "C" int srfx_tor_osem_subset(const float *lors, int64_t n, int64_t ld, co
                                nslab);
     if (rc)
         return rc;
+    if (binned_ok(p, flags, st)) {
+        bool done = false;
+        rc = binned_scatter(kOsem, p, st, &done);
+        if (rc || done)
+            return rc;
+    }
     if (nslab == 0 || n == 0)
         return launch<kOsem>(p, flags, st);
     void *ws = nullptr;

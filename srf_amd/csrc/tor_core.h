@@ -650,16 +650,14 @@ namespace {
 // voxels.  The gather keeps the decisions as per-voxel lane masks and sums in
 // the reference's order (rows outer, columns inner) with the arithmetic of
 // patch_walk; the scatter and the count decide from d2 - thr directly.
-//   KIND 0: returns sum w * src[idx]; 1: dst[idx] += w, amp carrying the
-//   scale (LDS: LDS atomics in dst's type, else FP32 global atomics);
-//   2: returns the count.
-//   LDS: 0 strided image; 1 LDS tile with unit column stride (idx.si = 1);
-//   2 LDS tile with unit row stride (idx.sj = 1).
-template <int KIND, int BX, int BY, int LDS, typename D>
+//   KIND 0: returns sum w * src[idx]; 1: dst[idx] += w with FP32 global
+//   atomics, amp carrying the scale; 2: returns the count.
+//   LDS (KIND 0): src is an LDS tile with unit column stride (idx.si = 1).
+template <int KIND, int BX, int BY, bool LDS>
 __device__ __forceinline__ float slice_box(const TorParams &p, const Event &ev, const Track &t,
-                                           const Cross &c, float amp, int s, float scale, int i_lo,
-                                           int i_hi, int j_lo, int j_hi, const PatchIdx &idx,
-                                           const float *src, D *dst)
+                                           const Cross &c, float amp, int s, int i_lo, int i_hi,
+                                           int j_lo, int j_hi, const PatchIdx &idx,
+                                           const float *src, float *dst)
 {
     constexpr int NC = BX * BY;
     const float eps = 1.0e-4f;
@@ -667,11 +665,6 @@ __device__ __forceinline__ float slice_box(const TorParams &p, const Event &ev, 
     const int jb0 = (int)ceilf((c.dy0 - t.dymax) * p.rfinter_y - eps);
     const int ib = max(i_lo, ib0), ie = min(i_hi, ib0 + t.nx - 1);
     const int jb = max(j_lo, jb0), je = min(j_hi, jb0 + t.ny - 1);
-    // LDS tiles have unit column (LDS 1) or row (LDS 2) stride: one address
-    // per box row (column), formed after the decisions (opaque, so not
-    // re-formed per voxel inside the branches), and the other index as an
-    // immediate offset
-    int row[BY], col[BX];
     // dt = d2 - thr of every candidate from its column and row terms; the
     // smallest |dt| decides whether the FP64 decision is needed at all
     float cx2[BX], cux[BX], rt2[BY], ruy[BY];
@@ -720,7 +713,10 @@ __device__ __forceinline__ float slice_box(const TorParams &p, const Event &ev, 
             for (int k = 0; k < NC; k++)
                 in[k] |= ((add >> k) & 1u) != 0;
         }
-        static_assert(LDS != 2, "gathers read x-fastest tiles");
+        // LDS tiles: one address per box row, formed after the decisions
+        // (opaque, so not re-formed per voxel inside the branches), and the
+        // column as an immediate offset
+        int row[BY];
 #pragma unroll
         for (int jj = 0; jj < BY; jj++)
             row[jj] = LDS ? opaque(idx(ib, jb + jj)) : 0;
@@ -790,11 +786,7 @@ __device__ __forceinline__ float slice_box(const TorParams &p, const Event &ev, 
                         const float w = voxel_weight(
                             ev, amp, voxel_dt(ev, voxel_offset(c.dx0, i, p.finter_x),
                                               voxel_offset(c.dy0, j, p.finter_y)));
-                        D *q = dst + idx(i, j);
-                        if constexpr (LDS != 0)
-                            atomicAdd(q, (D)w);
-                        else
-                            unsafeAtomicAdd(q, w);
+                        unsafeAtomicAdd(dst + idx(i, j), w);
                     }
                 }
             }
@@ -805,27 +797,11 @@ __device__ __forceinline__ float slice_box(const TorParams &p, const Event &ev, 
                 cnt += dt[k] < -kThrMargin ? 1.0f : 0.0f;
             return cnt;
         }
-        if constexpr (LDS == 2) {
-#pragma unroll
-            for (int ii = 0; ii < BX; ii++)
-                col[ii] = opaque(idx(ib + ii, jb));
-        } else {
-#pragma unroll
-            for (int jj = 0; jj < BY; jj++)
-                row[jj] = LDS ? opaque(idx(ib, jb + jj)) : 0;
-        }
 #pragma unroll
         for (int k = 0; k < NC; k++) {
-            if (dt[k] < -kThrMargin) {
-                const float w = voxel_weight(ev, amp, dt[k]);
-                D *q = dst + (LDS == 2   ? col[k % BX] + k / BX
-                              : LDS == 1 ? row[k / BX] + k % BX
-                                         : idx(ib + k % BX, jb + k / BX));
-                if constexpr (LDS != 0)
-                    atomicAdd(q, (D)w);
-                else
-                    unsafeAtomicAdd(q, w);
-            }
+            if (dt[k] < -kThrMargin)
+                unsafeAtomicAdd(dst + idx(ib + k % BX, jb + k / BX),
+                                voxel_weight(ev, amp, dt[k]));
         }
         return 0.0f;
     }
@@ -1045,10 +1021,10 @@ __device__ __forceinline__ float slice_box_image(const TorParams &p, const Event
         idx.sj = p.oy;
     }
     if (shape == 1)
-        return slice_box<KIND, NB, NB - 1, 0>(p, ev, t, c, amp, s, scale, i_lo, i_hi, j_lo,
-                                                  j_hi, idx, p.img, p.out);
-    return slice_box<KIND, NB, NB, 0>(p, ev, t, c, amp, s, scale, i_lo, i_hi, j_lo, j_hi,
-                                          idx, p.img, p.out);
+        return slice_box<KIND, NB, NB - 1, false>(p, ev, t, c, amp, s, i_lo, i_hi, j_lo, j_hi,
+                                                  idx, p.img, p.out);
+    return slice_box<KIND, NB, NB, false>(p, ev, t, c, amp, s, i_lo, i_hi, j_lo, j_hi, idx,
+                                          p.img, p.out);
 }
 
 // Walk the crossed slices s_first, s_first + rstep, ... <= s_last of an event
