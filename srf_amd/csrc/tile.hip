@@ -121,15 +121,17 @@ int launch_record_project(const TorParams &p, float4 *rec, uint32_t flags, hipSt
         return SRFX_OK;
     static const int kBlock[4] = {256, 64, 128, 256};
     const int block = kBlock[(flags >> SRFX_BLOCK_SHIFT) & 3u];
-    // no lanes-per-event flag: four lanes per event, the fastest measured
-    switch ((flags >> SRFX_LPE_SHIFT) & 3u) {
-    case 1:
+    // no lanes-per-event flag: four lanes per event, the fastest measured for
+    // large sets, 16 for sets that would leave the chip idle
+    static const int kLanes[4] = {0, 1, 4, 16};
+    int lanes = kLanes[(flags >> SRFX_LPE_SHIFT) & 3u];
+    if (lanes == 0)
+        lanes = lanes_per_event(p.n) == 16 ? 16 : 4;
+    if (lanes == 1)
         return launch_record_lpe<1>(p, rec, pout, block, st);
-    case 3:
+    if (lanes == 16)
         return launch_record_lpe<16>(p, rec, pout, block, st);
-    default:
-        return launch_record_lpe<4>(p, rec, pout, block, st);
-    }
+    return launch_record_lpe<4>(p, rec, pout, block, st);
 }
 
 // Count, scan (host: per tile; device: per event when slots are kept), fill,

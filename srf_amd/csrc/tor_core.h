@@ -1354,25 +1354,38 @@ int launch_slab_sum(const float *part, int nslab, int64_t n, float *out, hipStre
     return launch_status();
 }
 
-// Launch schedule from the flags: lanes per event (1, 4, 16) and block size
-// (64, 128, 256).  Kernels are specialised for the candidate box size
-// (3 or 4); the full-patch verification path and larger boxes use the
-// generic loops.
+// Lanes per event of a launch whose flags name none.  One event's walk is a
+// serial chain over its slices, so a small set takes as many lanes per event
+// as leave the chip about six waves per SIMD: 16 up to 24k events, 4 up to
+// 128k, then one.  Projection at 200 x 200 x 100 (4 mm tube, 530 ps), 1, 4 and
+// 16 lanes: 1000 events 127, 36 and 14 us; 16000 139, 43 and 27; 64000 138, 83
+// and 83; 250000 294, 294 and 281; without TOF at 250000 341, 495 and 638, so
+// one lane for large sets.  (Counts keep one: they check the walks.)
+inline int lanes_per_event(int64_t n)
+{
+    return n <= 24576 ? 16 : (n <= 131072 ? 4 : 1);
+}
+
+// Launch schedule from the flags: lanes per event (1, 4, 16; none:
+// lanes_per_event) and block size (64, 128, 256).  Kernels are specialised for
+// the candidate box size (3 or 4); the full-patch verification path and larger
+// boxes use the generic loops.
 template <int MODE>
 int launch(const TorParams &p, uint32_t flags, hipStream_t st)
 {
     if (p.n == 0)
         return SRFX_OK;
     static const int kBlock[4] = {256, 64, 128, 256};
+    static const int kLanes[4] = {0, 1, 4, 16};
     const int block = kBlock[(flags >> SRFX_BLOCK_SHIFT) & 3u];
-    switch ((flags >> SRFX_LPE_SHIFT) & 3u) {
-    case 2:
+    int lanes = kLanes[(flags >> SRFX_LPE_SHIFT) & 3u];
+    if (lanes == 0)
+        lanes = MODE == kCount ? 1 : lanes_per_event(p.n);
+    if (lanes == 4)
         return launch_lpe<MODE, 4>(p, block, st);
-    case 3:
+    if (lanes == 16)
         return launch_lpe<MODE, 16>(p, block, st);
-    default:
-        return launch_lpe<MODE, 1>(p, block, st);
-    }
+    return launch_lpe<MODE, 1>(p, block, st);
 }
 
 srfx_tor_model model_no_tof(float kw, int geo)
