@@ -346,11 +346,11 @@ int srfx_tor_plan_scales(srfx_tor_plan plan, float *out, void *stream);
  * own atomic, siddon.cu.cc:339-381; the ops compute what
  * srfx_siddon_backproject / _backproject_adjoint / _osem_subset compute for
  * the same LORs, with the same voxels and segment values, summed in another
- * order).  A plan cuts each LOR's walk into runs, one per image tile of
- * tx x ty x tz voxels it crosses (tx * ty * tz <= 8192: the scatter's tile is
- * FP64 in LDS), and lists the runs by tile; a scatter workgroup takes up to
- * `chunk` runs of one tile (0 = 2048), accumulates them in LDS and flushes
- * the tile with one atomic per non-zero voxel.  `block`: 64, 128 or 256
+ * order).  A plan lists each LOR in the image tiles of tx x ty x tz voxels it
+ * crosses (tx * ty * tz <= 8192: the scatter's tile is FP64 in LDS); a scatter
+ * workgroup takes up to `chunk` listings of one tile (0: 256 to 2048 by the
+ * plan's listings), accumulates them in LDS and flushes the tile with one
+ * atomic per non-zero voxel.  `block`: 64, 128 or 256
  * (0 = 256).  `sort` nonzero: the plan keeps a copy of its LORs sorted by
  * direction and position (a radix sort on the device), which its passes and
  * its OSEM projection read, so that the lanes of a wavefront trace nearly

@@ -76,33 +76,16 @@ __global__ __launch_bounds__(256) void bin_init(BinTables b, int nt, int64_t n)
 // it), 1024 tiles a round with a prefix sum of (listings, chunks).
 __global__ __launch_bounds__(kScanThreads) void bin_scan(BinTables b, TileGeom g, int nt)
 {
-    constexpr int W = kScanThreads / 64;
-    __shared__ long long wsum[W];
     const int nw = g.nwx * g.nwy;
-    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
     long long carry = 0; // listings | chunks << 40
     for (int q0 = 0; q0 < nt; q0 += kScanThreads) {
         const int q = q0 + (int)threadIdx.x;
         const int t = q < nt ? (q % g.nslab) * nw + q / g.nslab : 0;
         const int c = q < nt ? b.cnt[t] : 0;
         const int nch = (c + kBinChunk - 1) / kBinChunk;
-        const long long v = (long long)c | ((long long)nch << 40);
-        long long inc = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const long long u = __shfl_up(inc, d, 64);
-            inc += lane >= d ? u : 0;
-        }
-        if (lane == 63)
-            wsum[wv] = inc;
-        __syncthreads();
-        long long before = carry, total = 0;
-        for (int k = 0; k < W; k++) {
-            before += k < wv ? wsum[k] : 0;
-            total += wsum[k];
-        }
-        __syncthreads();
-        const long long ex = before + inc - v;
+        long long total;
+        const long long ex =
+            carry + block_scan<kScanThreads>((long long)c | ((long long)nch << 40), total);
         const long long o = ex & ((1ll << 40) - 1);
         const int ch = (int)(ex >> 40);
         if (q < nt) {
@@ -246,8 +229,6 @@ int launch_bin_box(const TorParams &p, const TileGeom &g, const BinTables &b, in
     }
 }
 
-size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-
 } // namespace
 
 // Weights (event, voxel) from which an untiled scatter runs binned.  The direct
@@ -281,13 +262,7 @@ bool binned_ok(const TorParams &p, uint32_t flags, hipStream_t st)
     const TileGeom g = bin_geom(p);
     if ((int64_t)g.nwx * g.nwy * g.nslab >= (1 << 20))
         return false;
-    // a captured call keeps the kernels that need no workspace
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return cap == hipStreamCaptureStatusNone;
+    return workspace_ok(st);
 }
 
 int binned_scatter(int mode, const TorParams &p, hipStream_t st, bool *done)

@@ -97,9 +97,58 @@ inline bool slab_schedule(uint32_t flags, int &nslab, int &interleave)
     }
 }
 
+// Next work item of a persistent block (the same value in every thread).
+static __device__ __forceinline__ int next_item(unsigned *counter)
+{
+    __shared__ int item;
+    if (threadIdx.x == 0)
+        item = (int)atomicAdd(counter, 1u);
+    __syncthreads();
+    const int c = __builtin_amdgcn_readfirstlane(item);
+    __syncthreads();
+    return c;
+}
+
+// Exclusive prefix sum of v over a workgroup of T threads (a multiple of 64);
+// total receives the sum.  Every thread calls it.
+template <int T>
+static __device__ __forceinline__ long long block_scan(long long v, long long &total)
+{
+    __shared__ long long wsum[T / 64];
+    const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+    long long inc = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const long long u = __shfl_up(inc, d, 64);
+        inc += lane >= d ? u : 0;
+    }
+    if (lane == 63)
+        wsum[wv] = inc;
+    __syncthreads();
+    long long before = 0;
+    total = 0;
+    for (int k = 0; k < T / 64; k++) {
+        before += k < wv ? wsum[k] : 0;
+        total += wsum[k];
+    }
+    __syncthreads();
+    return before + inc - v;
+}
+
+// A workgroup's share of a tile: entries start .. start + count - 1 of a list.
+struct TileSpan {
+    int tile, start, count;
+};
+
 // Stream-ordered device workspace: allocated from the device's default memory
 // pool (kept by the pool between calls) and released on the same stream.
 int ws_alloc(void **ptr, size_t bytes, hipStream_t st);
 int ws_free(void *ptr, hipStream_t st);
+
+inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Whether st may be given work that takes a workspace (a captured call keeps
+// to the kernels that need none).
+bool workspace_ok(hipStream_t st);
 
 } // namespace srfx

@@ -1,68 +1,65 @@
-// Siddon ray-driven projector for CDNA4 (gfx950): the untiled ops, one lane
-// per LOR (siddon.cu.cc:424-675).  Ray setup, the walk and its precision are
-// in siddon_core.h.
+// Siddon ray-driven projector for CDNA4 (gfx950): the untiled ops
+// (siddon.cu.cc:424-675).  Ray setup, the walks and their precision are in
+// siddon_core.h.
 //
 // Unlike the reference, a ray whose start voxel falls outside the grid is
 // skipped (the reference indexes out of bounds there), and the walk is capped
 // at gx+gy+gz+3 steps; both only affect degenerate rays.
-#include "siddon_core.h"
+#include "siddon_binned.h"
 
 namespace srfx {
 namespace {
 
-template <int MODE>
+// L lanes per ray (walk_ray).  The mode's reference semantics: projection,
+// A^T(1 / v) over v > 0, the map likewise without TOF, plain adjoint, and the
+// OSEM pass (both).
+template <int MODE, int L, bool TOF>
 __global__ __launch_bounds__(256) void siddon_kernel(SidParams p)
 {
-    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int R = 256 / L; // rays of the workgroup (ray_sum)
+    const int64_t e = (int64_t)blockIdx.x * R + (int)threadIdx.x % R;
+    const int sub = (int)threadIdx.x / R;
+    const bool valid = e < p.n;
+    SidRay r;
+    r.tend = -1.0;
+    r.weight = 0.0f;
+    r.t_tof = 0.0;
+    if (valid) {
+        Walk w;
+        setup_walk<MODE>(p, e, w);
+        if (w.ok)
+            make_ray(w, r);
+    }
+    float scale = 0.0f;
+    if (MODE == kProj || MODE == kOsem) {
+        const float pv = ray_sum<L>(r.tend > 0.0 ? gather_ray<TOF, L>(p, r, sub) : 0.0f);
+        if (MODE == kProj) {
+            if (valid && sub == 0)
+                p.out[e] = pv;
+            return;
+        }
+        scale = pv > 0.0f ? 1.0f / pv : 0.0f;
+    } else if (valid) {
+        const float v = p.val[e];
+        scale = MODE == kAdj ? v : (v > 0.0f ? 1.0f / v : 0.0f);
+    }
+    if (scale != 0.0f && r.tend > 0.0)
+        scatter_ray<TOF, L>(p, r, sub, scale);
+}
+
+__global__ __launch_bounds__(256) void siddon_count(SidParams p)
+{
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int cnt = 0;
     if (e < p.n) {
         Walk w;
-        setup_walk<MODE>(p, e, w);
-        const bool tof = (MODE != kMap) && p.use_tof;
-        if (MODE == kProj) {
-            float pv = 0.0f;
-            if (w.ok)
-                pv = tof ? walk<0, true>(p, w, 0.0f, nullptr) : walk<0, false>(p, w, 0.0f, nullptr);
-            p.out[e] = pv;
-        } else if (MODE == kBack || MODE == kMap) {
-            float v = p.val[e];
-            if (w.ok && v > 0.0f) {
-                if (tof)
-                    walk<1, true>(p, w, 1.0f / v, nullptr);
-                else
-                    walk<1, false>(p, w, 1.0f / v, nullptr);
-            }
-        } else if (MODE == kAdj) {
-            float g = p.val[e];
-            if (w.ok && g != 0.0f) {
-                if (tof)
-                    walk<1, true>(p, w, g, nullptr);
-                else
-                    walk<1, false>(p, w, g, nullptr);
-            }
-        } else if (MODE == kOsem) {
-            if (w.ok) {
-                float pv = tof ? walk<0, true>(p, w, 0.0f, nullptr)
-                               : walk<0, false>(p, w, 0.0f, nullptr);
-                if (pv > 0.0f) {
-                    if (tof)
-                        walk<1, true>(p, w, 1.0f / pv, nullptr);
-                    else
-                        walk<1, false>(p, w, 1.0f / pv, nullptr);
-                }
-            }
-        } else { // kCount
-            if (w.ok) {
-                if (tof)
-                    walk<2, true>(p, w, 0.0f, &cnt);
-                else
-                    walk<2, false>(p, w, 0.0f, &cnt);
-            }
-            if (p.nnz)
-                p.nnz[e] = cnt;
-        }
+        setup_walk<kCount>(p, e, w);
+        if (w.ok)
+            cnt = p.use_tof ? count_segments<true>(p, w) : count_segments<false>(p, w);
+        if (p.nnz)
+            p.nnz[e] = cnt;
     }
-    if (MODE == kCount && p.nnz_total) {
+    if (p.nnz_total) {
         unsigned long long c = (unsigned long long)cnt;
         for (int off = 32; off > 0; off >>= 1)
             c += __shfl_down(c, off, 64);
@@ -71,8 +68,39 @@ __global__ __launch_bounds__(256) void siddon_kernel(SidParams p)
     }
 }
 
-int setup(SidParams &p, const float *lors, int64_t n, int64_t ld, const srfx_grid &g,
-          float tof_bin, float tof_sigma2)
+template <int MODE, int L>
+int launch_lanes(const SidParams &p, hipStream_t st)
+{
+    const dim3 grid(blocks_for(p.n * L, 256)), block(256);
+    if constexpr (MODE != kMap) {
+        if (p.use_tof) {
+            hipLaunchKernelGGL((siddon_kernel<MODE, L, true>), grid, block, 0, st, p);
+            return launch_status();
+        }
+    }
+    hipLaunchKernelGGL((siddon_kernel<MODE, L, false>), grid, block, 0, st, p);
+    return launch_status();
+}
+
+template <int MODE>
+int launch(const SidParams &p, hipStream_t st)
+{
+    if (p.n == 0)
+        return SRFX_OK;
+    switch (lanes_per_ray(p.n)) {
+    case 16:
+        return launch_lanes<MODE, 16>(p, st);
+    case 4:
+        return launch_lanes<MODE, 4>(p, st);
+    default:
+        return launch_lanes<MODE, 1>(p, st);
+    }
+}
+
+} // namespace
+
+int siddon_setup(SidParams &p, const float *lors, int64_t n, int64_t ld, const srfx_grid &g,
+                 float tof_bin, float tof_sigma2)
 {
     if (n < 0 || (n > 0 && (!lors || ld < n)) || !grid_ok(g))
         return SRFX_EINVAL;
@@ -95,16 +123,6 @@ int setup(SidParams &p, const float *lors, int64_t n, int64_t ld, const srfx_gri
     return SRFX_OK;
 }
 
-template <int MODE>
-int launch(const SidParams &p, hipStream_t st)
-{
-    if (p.n == 0)
-        return SRFX_OK;
-    hipLaunchKernelGGL(siddon_kernel<MODE>, dim3(blocks_for(p.n, 256)), dim3(256), 0, st, p);
-    return launch_status();
-}
-
-} // namespace
 } // namespace srfx
 
 using namespace srfx;
@@ -115,7 +133,7 @@ extern "C" int srfx_siddon_project(const float *lors, int64_t n, int64_t ld, con
 {
     (void)flags;
     SidParams p;
-    int rc = setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
+    int rc = siddon_setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
     if (rc)
         return rc;
     if (n > 0 && (!image || !proj))
@@ -130,7 +148,7 @@ static int sid_scatter(int mode, const float *lors, int64_t n, int64_t ld, const
                        uint32_t flags, void *stream)
 {
     SidParams p;
-    int rc = setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
+    int rc = siddon_setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
     if (rc)
         return rc;
     if (!image || (n > 0 && !vals))
@@ -141,6 +159,12 @@ static int sid_scatter(int mode, const float *lors, int64_t n, int64_t ld, const
         return rc;
     p.val = vals;
     p.out = image;
+    if (siddon_binned_ok(p, st)) {
+        bool done = false;
+        rc = siddon_binned_scatter(mode, p, st, &done);
+        if (rc || done)
+            return rc;
+    }
     switch (mode) {
     case kBack:
         return launch<kBack>(p, st);
@@ -180,7 +204,7 @@ extern "C" int srfx_siddon_osem_subset(const float *lors, int64_t n, int64_t ld,
                                        float tof_sigma2, float *bp, uint32_t flags, void *stream)
 {
     SidParams p;
-    int rc = setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
+    int rc = siddon_setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
     if (rc)
         return rc;
     if (!bp || (n > 0 && !image))
@@ -191,6 +215,12 @@ extern "C" int srfx_siddon_osem_subset(const float *lors, int64_t n, int64_t ld,
         return rc;
     p.img = image;
     p.out = bp;
+    if (siddon_binned_ok(p, st)) {
+        bool done = false;
+        rc = siddon_binned_scatter(kOsem, p, st, &done);
+        if (rc || done)
+            return rc;
+    }
     return launch<kOsem>(p, st);
 }
 
@@ -199,10 +229,14 @@ extern "C" int srfx_siddon_count_nnz(const float *lors, int64_t n, int64_t ld, s
                                      uint64_t *nnz_total, void *stream)
 {
     SidParams p;
-    int rc = setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
+    int rc = siddon_setup(p, lors, n, ld, grid, tof_bin, tof_sigma2);
     if (rc)
         return rc;
     p.nnz = nnz_per_event;
     p.nnz_total = (unsigned long long *)nnz_total;
-    return launch<kCount>(p, (hipStream_t)stream);
+    if (p.n == 0)
+        return SRFX_OK;
+    hipLaunchKernelGGL(siddon_count, dim3(blocks_for(p.n, 256)), dim3(256), 0,
+                       (hipStream_t)stream, p);
+    return launch_status();
 }

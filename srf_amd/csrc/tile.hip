@@ -283,11 +283,6 @@ done:
     return rc;
 }
 
-size_t align256(size_t b)
-{
-    return (b + 255) & ~(size_t)255;
-}
-
 // Whether plans of this tile shape and event count can be built as a set
 // (their list entries carry spans).
 bool set_buildable(const TileGeom &g, int64_t n, bool keep_slots)

@@ -29,6 +29,7 @@
 #include <atomic>
 #include <vector>
 
+#include "chunk_sort.h"
 #include "tor_core.h"
 
 namespace srfx {
@@ -1056,118 +1057,30 @@ __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom
     __syncthreads();
 }
 
-// Next work item of a persistent block (the same value in every thread).
-__device__ __forceinline__ int next_item(unsigned *counter)
-{
-    __shared__ int item;
-    if (threadIdx.x == 0)
-        item = (int)atomicAdd(counter, 1u);
-    __syncthreads();
-    const int c = __builtin_amdgcn_readfirstlane(item);
-    __syncthreads();
-    return c;
-}
-
-// The lanes of the wave whose v (0 <= v < 64) equals this lane's: one ballot
-// per bit of v.  Call with every lane of the wave active.
-__device__ __forceinline__ uint64_t lanes_with(int v)
-{
-    uint64_t m = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 6; b++) {
-        const bool bit = (v >> b) & 1;
-        const uint64_t bal = __ballot(bit);
-        m &= bit ? bal : ~bal;
-    }
-    return m;
-}
-
 // Plan build, after the fill pass: order each chunk's listings by the number
-// of slices they walk in the tile, longest first (a counting sort in LDS), so
-// that the consecutive listings a wave of the scatter takes walk about as
-// many slices each.  Inside a bucket the listings keep their order within a
-// wave and the waves their order of arrival, which with coalesced reads
-// keeps roughly the fill order.  The lanes of a wave with the same key count
-// and take their positions together: one LDS atomic per key and wave, the
-// lowest such lane's, instead of one per lane on a few shared counters.
-// With spans the slice counts come from the entries (the fill pass wrote
-// them) instead of the walk records.  One workgroup per chunk, 256 threads;
-// LDS: 33 counters and `chunk` ints.  Needs ch.count <= 16 * blockDim.x.
+// of slices they walk in the tile, longest first, so that the consecutive
+// listings a wave of the scatter takes walk about as many slices each.  With
+// spans the slice counts come from the entries (the fill pass wrote them)
+// instead of the walk records.  One workgroup per chunk, 256 threads; LDS: 33
+// counters and `chunk` ints.  Needs ch.count <= 16 * blockDim.x.
 template <bool SPANS>
 __device__ __forceinline__ void sort_chunk(const TorParams &p, const TileGeom &g,
                                            const TileChunk &ch, int *__restrict__ list,
                                            const float4 *__restrict__ rec, int *sh)
 {
-    constexpr int kBuckets = 32, kPer = 16;
-    int *cnt = sh, *ord = sh + kBuckets + 1;
-    const int lane = (int)threadIdx.x & 63;
-    for (int i = threadIdx.x; i <= kBuckets; i += blockDim.x)
-        cnt[i] = 0;
-    __syncthreads();
-    // per entry: its key (-1: no entry), event, and its rank among the wave's
-    // lanes with the same key | the first such lane << 6 | their number << 12
-    int key[kPer], ev[kPer], grp[kPer];
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        key[r] = -1;
-        ev[r] = 0;
-        grp[r] = 0;
-        if (r * (int)blockDim.x >= ch.count)
-            continue; // the same for every lane of the workgroup
-        const int j = r * (int)blockDim.x + (int)threadIdx.x; // coalesced reads
-        if (j < ch.count) {
-            ev[r] = list[ch.start + j];
-            int s0, s1;
-            if (SPANS) {
-                // the fill pass put the listing's slices in the entry
-                s0 = (ev[r] >> kSpanEventBits) & 15;
-                s1 = (int)((unsigned)ev[r] >> (kSpanEventBits + 4));
-            } else {
-                Event e;
-                Track t;
-                unpack_walk(p, rec, ev[r], e, t);
-                listing_slices(p, tile_box(p, g, ch.tile), e, t, s0, s1);
-            }
-            // longest first: bucket 0 holds the longest walks
-            key[r] = kBuckets - 1 - min(max(s1 - s0 + 1, 0), kBuckets - 1);
+    chunk_sort(list + ch.start, ch.count, sh, [&](int ent) {
+        int s0, s1;
+        if (SPANS) {
+            s0 = (ent >> kSpanEventBits) & 15;
+            s1 = (int)((unsigned)ent >> (kSpanEventBits + 4));
+        } else {
+            Event e;
+            Track t;
+            unpack_walk(p, rec, ent, e, t);
+            listing_slices(p, tile_box(p, g, ch.tile), e, t, s0, s1);
         }
-        const uint64_t m = lanes_with(key[r] + 1);
-        const int rank = (int)__builtin_amdgcn_mbcnt_hi(
-            (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-        const int n = __popcll(m);
-        grp[r] = rank | (__builtin_ctzll(m) << 6) | (n << 12);
-        if (key[r] >= 0 && rank == 0)
-            atomicAdd(&cnt[key[r]], n);
-    }
-    __syncthreads();
-    // exclusive prefix of the bucket counts, by the first wave
-    if (threadIdx.x < 64) {
-        const int c = lane < kBuckets ? cnt[lane] : 0;
-        int v = c;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int u = __shfl_up(v, d, 64);
-            v += lane >= d ? u : 0;
-        }
-        if (lane < kBuckets)
-            cnt[lane] = v - c;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kPer; r++) {
-        if (r * (int)blockDim.x >= ch.count)
-            continue;
-        const int rank = grp[r] & 63;
-        int base = 0;
-        if (key[r] >= 0 && rank == 0)
-            base = atomicAdd(&cnt[key[r]], grp[r] >> 12);
-        base = __shfl(base, (grp[r] >> 6) & 63, 64);
-        if (key[r] >= 0)
-            ord[base + rank] = ev[r];
-    }
-    __syncthreads();
-    for (int j = threadIdx.x; j < ch.count; j += blockDim.x)
-        list[ch.start + j] = ord[j];
+        return s1 - s0 + 1;
+    });
 }
 
 __global__ __launch_bounds__(256) void sort_chunks(TorParams p, TileGeom g,

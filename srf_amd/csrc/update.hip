@@ -101,6 +101,16 @@ int ws_free(void *ptr, hipStream_t st)
     return hipFreeAsync(ptr, st) == hipSuccess ? SRFX_OK : SRFX_ELAUNCH;
 }
 
+bool workspace_ok(hipStream_t st)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cap == hipStreamCaptureStatusNone;
+}
+
 } // namespace srfx
 
 using namespace srfx;

@@ -268,18 +268,18 @@ class TorPlan:
             pass
 
 
-DEFAULT_SIDDON_TILE = (16, 16, 16)
-DEFAULT_SIDDON_CHUNK = 2048
+DEFAULT_SIDDON_TILE = (16, 16, 8)
+DEFAULT_SIDDON_CHUNK = 0  # by the plan's listings
 
 
 class SiddonPlan:
     """Tiled Siddon backprojection over a fixed LOR set (srfx_siddon_plan_*).
 
-    The plan cuts each LOR's walk (siddon.cu.cc:293-331) into runs, one per
-    image tile of ``tile`` voxels it crosses, and lists the runs by tile; its
-    backprojections accumulate each tile in LDS and flush it with coalesced
-    atomics.  Same voxels and segment values as the untiled ops
-    (siddon.cc:28-43 semantics), summed in another order.  OSEM reuses one
+    The plan lists every LOR in each image tile of ``tile`` voxels its walk
+    (siddon.cu.cc:293-331) crosses; its backprojections accumulate each tile
+    in LDS and flush it with coalesced atomics.  Same voxels and segment
+    values as the untiled ops (siddon.cc:28-43 semantics), summed in another
+    order.  OSEM reuses one
     plan per subset for every iteration.
 
     The plan keeps a reference to the LOR tensor (7 x N SoA: x1..z2, tof): it
@@ -353,15 +353,15 @@ class SiddonPlan:
         return int(a.value), int(b.value)
 
     def device_bytes(self):
-        """Device memory held by the plan: 48 bytes per run, 52 per LOR (ray
-        record, projection buffer), 16 per chunk, 8 per tile, and with the
-        sorted LOR stream 32 more per LOR (sorted copy, permutation) and the
-        build's sort buffers (24 per LOR)."""
+        """Device memory held by the plan: 4 bytes per (LOR, tile) listing, 84
+        per LOR (ray record, projection buffer), 16 per chunk, 8 per tile, and
+        with the sorted LOR stream 32 more per LOR (sorted copy, permutation)
+        and the build's sort buffers (24 per LOR)."""
         nr, nc = self.info()
         nt = 1
         for g, t in zip(self.grid, self.tile):
             nt *= -(-g // min(t, g))
-        return (48 * nr + 52 * self.n + 16 * nc + 8 * nt
+        return (4 * nr + 84 * self.n + 16 * nc + 8 * nt
                 + (56 * self.n if self.sorted else 0))
 
     def _image(self, image, name):

@@ -25,7 +25,8 @@ def _events(n, size, seed, steep=False):
     t = r.uniform(0.5, 1.0, n)[:, None] * size[2]
     p1, p2 = mid - d * t, mid + d * t
     pc = p1 + r.uniform(0.3, 0.7, n)[:, None] * (p2 - p1)
-    lors = np.vstack([p1.T, p2.T, pc.T, r.uniform(0.7, 1.2, n)[None]]).astype(np.float32)
+    lors = np.ascontiguousarray(
+        np.vstack([p1.T, p2.T, pc.T, r.uniform(0.7, 1.2, n)[None]]), np.float32)
     return torch.from_numpy(lors).to(DEV), torch.from_numpy(
         r.uniform(0.5, 2.0, n).astype(np.float32)).to(DEV)
 
