@@ -341,6 +341,38 @@ int srfx_tor_plan_osem_subset(srfx_tor_plan plan, const float *image, srfx_grid 
  * output is the tensor of op "Projection", tor.cc:122-128). */
 int srfx_tor_plan_scales(srfx_tor_plan plan, float *out, void *stream);
 
+/* LOR preprocessing of the TOR model (preprocess/function/on_tor_lors.py:70-77,
+ * 137-262), in two calls around the allocation of the groups.  rows: n list-mode
+ * rows x1..z2, tof (7 columns) or pair rows x1..z2 (6), float or (f64) double,
+ * element (e, c) at rows[e * row_stride + c * col_stride].
+ * _count: rows by dominant axis and direction into totals[6] = {x, x swapped, y,
+ * y swapped, z, z swapped} (device), with work[6 * ceil(n / 1024)] (device).
+ * _fill: group a (0 x, 1 y, 2 z) of N_a = totals[2 a] + totals[2 a + 1] rows
+ * into out[a], rows of ld[a] >= N_a floats: p1, p2, (7 columns: TOF centre,)
+ * sigma2 factor in the group frame, rows with a non-negative difference along
+ * the axis in input order, then the swapped ones.  cut (7 columns): end points
+ * further than `limit` mm from the TOF centre are cut to it.  order (nullable,
+ * and each entry): the input row of each output row.  out, ld and order are
+ * host arrays of three.  FP64 in the reference's order of operations, rounded to
+ * float once. */
+int srfx_split_lors_count(const void *rows, int64_t n, int64_t row_stride, int64_t col_stride,
+                          int32_t f64, int32_t *work, int64_t *totals, void *stream);
+int srfx_split_lors_fill(const void *rows, int64_t n, int64_t row_stride, int64_t col_stride,
+                         int32_t f64, int32_t ncols, int32_t cut, double limit,
+                         const int32_t *work, const int64_t *totals, float *const *out,
+                         const int64_t *ld, int64_t *const *order, void *stream);
+
+/* Locality order of a group's events (no reference counterpart): order[j] = the
+ * event at position j when every OSEM subset [k n / K, (k + 1) n / K) is sorted,
+ * stably, by coarse TOF-centre position along the slice axis (bins of zc_bin
+ * mm), then by the Morton interleave of the two slopes (slope_bin) and the
+ * crossing with the plane z = center_z (pos_bin mm).  soa: [ncols >= 9, n], row
+ * stride ld; out (nullable): the reordered [ncols, n].  Stream-ordered
+ * workspace from the device's memory pool. */
+int srfx_locality_sort(const float *soa, int64_t n, int64_t ld, int32_t ncols,
+                       int32_t nb_subsets, double center_z, double zc_bin, double slope_bin,
+                       double pos_bin, float *out, int64_t *order, void *stream);
+
 /* Tiled Siddon backprojection over a fixed LOR set (no counterpart in the
  * reference, whose BackRayTracing adds every segment to the image with its
  * own atomic, siddon.cu.cc:339-381; the ops compute what

@@ -99,6 +99,7 @@ _I64 = ctypes.c_int64
 _U32 = ctypes.c_uint32
 _F = ctypes.c_float
 _I32 = ctypes.c_int32
+_D = ctypes.c_double
 
 # name -> argtypes (all return int)
 _PROTOS = {
@@ -146,6 +147,10 @@ _PROTOS = {
     "srfx_siddon_plan_backproject_adjoint": [_P, _P, _P, _U32, _P],
     "srfx_siddon_plan_osem_subset": [_P, _P, _P, _P, _U32, _P],
     "srfx_siddon_plan_projection": [_P, _P, _P],
+    "srfx_split_lors_count": [_P, _I64, _I64, _I64, _I32, _P, _P, _P],
+    "srfx_split_lors_fill": [_P, _I64, _I64, _I64, _I32, _I32, _I32, _D, _P, _P,
+                             ctypes.POINTER(_P), ctypes.POINTER(_I64), ctypes.POINTER(_P), _P],
+    "srfx_locality_sort": [_P, _I64, _I64, _I32, _I32, _D, _D, _D, _D, _P, _P, _P],
 }
 
 _lib = None

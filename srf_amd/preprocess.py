@@ -13,8 +13,17 @@ structure-of-arrays float32 tensors in the group frame, ready for the ops:
 Row order inside a group is the reference's: ascending event index
 (np.intersect1d) for rows with d_axis >= 0, then those with d_axis < 0
 (SwapPointsOrder).  ``order`` maps output rows to input rows.
+
+float32 and float64 rows on a GPU go through the HIP kernels
+(srfx_split_lors_*, srfx_locality_sort), which give the same bits; other rows
+(host tensors, other types, rows that require a gradient) through the torch
+operations below.
 """
+import ctypes
+
 import torch
+
+from . import _lib
 
 AXES = ("x", "y", "z")
 GAUSSIAN_FACTOR = 2.35482005  # on_tor_lors.py:220
@@ -91,8 +100,51 @@ def _as64(lors, ncols):
     return lors.to(torch.float64)
 
 
+def _native(t):
+    return (type(t) is torch.Tensor and t.device.type == "cuda" and not t.requires_grad
+            and t.dim() == 2 and t.numel() > 0)
+
+
+SPLIT_ROWS = 1024  # rows per workgroup of srfx_split_lors_count
+
+
+def _split(rows, ncols, cut, limit, return_order):
+    """recon_process (ncols 7) or map_process (6) of float32 / float64 device
+    rows through srfx_split_lors_*: one count, the group sizes read back, one
+    fill."""
+    n, dev = rows.shape[0], rows.device
+    with torch.cuda.device(dev):
+        st = torch.cuda.current_stream().cuda_stream
+        src = (rows.data_ptr(), n, rows.stride(0), rows.stride(1),
+               1 if rows.dtype == torch.float64 else 0)
+        work = torch.empty(6 * -(-n // SPLIT_ROWS), dtype=torch.int32, device=dev)
+        totals = torch.empty(6, dtype=torch.int64, device=dev)
+        _lib.call("srfx_split_lors_count", *src, work.data_ptr(), totals.data_ptr(), st)
+        t = totals.tolist()
+        sizes = [t[0] + t[1], t[2] + t[3], t[4] + t[5]]
+        k = 10 if ncols == 7 else 7
+        out = [torch.empty((k, m), dtype=torch.float32, device=dev) for m in sizes]
+        order = [torch.empty(m, dtype=torch.int64, device=dev) if return_order else None
+                 for m in sizes]
+        ptrs = (ctypes.c_void_p * 3)(*[o.data_ptr() for o in out])
+        lds = (ctypes.c_int64 * 3)(*sizes)
+        ords = (ctypes.c_void_p * 3)(*[None if o is None else o.data_ptr() for o in order])
+        _lib.call("srfx_split_lors_fill", *src, ncols, 1 if cut else 0, float(limit),
+                  work.data_ptr(), totals.data_ptr(), ptrs, lds, ords, st)
+    out = dict(zip(AXES, out))
+    return (out, dict(zip(AXES, order))) if return_order else out
+
+
+def _splittable(lors, ncols):
+    return (_native(lors) and lors.shape[1] == ncols and lors.shape[0] < 2 ** 31
+            and lors.dtype in (torch.float32, torch.float64))
+
+
 def recon_process(lors, tof_res, return_order=False):
     """on_tor_lors.py:251-262.  lors: [N, 7] rows (x1, y1, z1, x2, y2, z2, tof)."""
+    if _splittable(lors, 7):
+        return _split(lors, 7, tof_res < 10000, tof_res * 0.15 / GAUSSIAN_FACTOR * 3,
+                      return_order)
     lors = _as64(lors, 7)
     lors = torch.cat([lors, sigma2_factor(lors)[:, None]], 1)
     masks = dominant_masks(lors)
@@ -109,6 +161,8 @@ def recon_process(lors, tof_res, return_order=False):
 
 def map_process(lors, return_order=False):
     """on_tor_lors.py:243-248.  lors: [N, 6] rows (x1, y1, z1, x2, y2, z2)."""
+    if _splittable(lors, 6):
+        return _split(lors, 6, False, 0.0, return_order)
     lors = _as64(lors, 6)
     lors = torch.cat([lors, sigma2_factor(lors)[:, None]], 1)
     masks = dominant_masks(lors)
@@ -156,10 +210,36 @@ def locality_key(soa, center_z, zc_bin=40.0, slope_bin=0.04, pos_bin=6.0):
     return (zc << 32) | m
 
 
+# locality_key's bins: TOF centre (mm), slopes, crossing point (mm)
+ZC_BIN, SLOPE_BIN, POS_BIN = 40.0, 0.04, 6.0
+
+
+def _sortable(soa, nb_subsets):
+    return (_native(soa) and soa.dtype == torch.float32 and soa.shape[0] >= 9
+            and soa.shape[1] < 2 ** 31 - 1 and 1 <= nb_subsets <= 1 << 24
+            and soa.stride(1) == 1 and soa.stride(0) >= soa.shape[1])
+
+
+def _locality_sort(soa, nb_subsets, center_z, gather):
+    """(reordered group or None, order) through srfx_locality_sort."""
+    with torch.cuda.device(soa.device):
+        n = soa.shape[1]
+        out = torch.empty((soa.shape[0], n), dtype=soa.dtype,
+                          device=soa.device) if gather else None
+        order = torch.empty(n, dtype=torch.int64, device=soa.device)
+        _lib.call("srfx_locality_sort", soa.data_ptr(), n, soa.stride(0), soa.shape[0],
+                  int(nb_subsets), float(center_z), ZC_BIN, SLOPE_BIN, POS_BIN,
+                  out.data_ptr() if gather else None, order.data_ptr(),
+                  torch.cuda.current_stream().cuda_stream)
+    return out, order
+
+
 def locality_order(soa, nb_subsets, center_z=0.0):
     """Permutation of a group's events that sorts each OSEM subset's rows
     [k N / K, (k+1) N / K) by locality_key and leaves subset membership
     unchanged."""
+    if _sortable(soa, nb_subsets):
+        return _locality_sort(soa, nb_subsets, center_z, False)[1]
     n = soa.shape[1]
     key = locality_key(soa, center_z)
     order = torch.empty(n, dtype=torch.int64, device=soa.device)
@@ -176,6 +256,9 @@ def reorder_groups(groups, nb_subsets, centers=None):
     out, orders = {}, {}
     for a, soa in groups.items():
         cz = 0.0 if centers is None else centers[a]
+        if _sortable(soa, nb_subsets):
+            out[a], orders[a] = _locality_sort(soa, nb_subsets, cz, True)
+            continue
         o = locality_order(soa, nb_subsets, cz)
         out[a] = soa[:, o].contiguous()
         orders[a] = o
