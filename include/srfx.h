@@ -67,7 +67,10 @@ enum srfx_status {
  * OSEM pass; ~2.4e6 weights and up) runs binned: its events are listed by image
  * tile on the device and every tile accumulated in LDS, with a stream-ordered
  * workspace of up to 256 MiB from the device's memory pool (a stream under
- * capture, or a failed allocation, keeps the kernels without workspace). */
+ * capture, or a failed allocation, keeps the kernels without workspace).
+ * Likewise the projection of more than 131072 events over an image of 10 MB
+ * and up (4 MB with tubes wider than four voxels) walks the events in a
+ * locality order formed on the device (up to 156 MiB of workspace). */
 #define SRFX_LPE_SHIFT 4
 #define SRFX_LPE_1 (1u << SRFX_LPE_SHIFT)
 #define SRFX_LPE_4 (2u << SRFX_LPE_SHIFT)

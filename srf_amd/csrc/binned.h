@@ -15,4 +15,8 @@ bool binned_ok(const TorParams &p, uint32_t flags, hipStream_t st);
 // was and the caller runs the direct kernels.
 int binned_scatter(int mode, const TorParams &p, hipStream_t st, bool *done);
 
+// The untiled projection (p.img, p.out set) of a large event set in locality
+// order.  done as above.
+int sorted_project(const TorParams &p, uint32_t flags, hipStream_t st, bool *done);
+
 } // namespace srfx

@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "binned.h"
+#include "locality.h"
 #include "tile_core.h"
 
 namespace srfx {
@@ -348,6 +349,112 @@ int binned_scatter(int mode, const TorParams &p, hipStream_t st, bool *done)
             rc = launch_bin_box<kOsem>(q, g, b, cus, st);
             break;
         }
+    }
+    *done = true;
+    const int rf = ws_free(ws, st);
+    return rc ? rc : rf;
+}
+
+namespace {
+
+// Walk records of a set's events at their places in its locality order, the
+// event's number in the record's value slot.  FP64 event set-up once per event.
+__global__ __launch_bounds__(256) void sorted_place_kernel(TorParams p, LocalityOrder o,
+                                                           float4 *rec)
+{
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= p.n)
+        return;
+    RawEvent r;
+    fetch_event<kProj>(p, e, r);
+    const ExactGeom eg = exact_geom(p, r);
+    Event ev;
+    Track t;
+    const bool valid = init_event<kProj>(p, r, eg, ev);
+    if (valid)
+        make_track(p, ev, eg, r, t);
+    const int64_t j = (int64_t)atomicAdd(&o.cursor[o.key[e]], 1u);
+    pack_walk(p, r, ev, t, valid, rec, j);
+    reinterpret_cast<int *>(rec)[4 * kWalkHead * j + kWalkValue] = (int)e;
+}
+
+// The projection of events in locality order from their records, as
+// record_proj_kernel's (four lanes per event, the 16 events of a wave on the
+// same slices at the same time, so that their gathers share cache lines), to the
+// events' own numbers.  FRAME: p.img is a contiguous op frame of p.img_bytes.
+template <int NB, bool FRAME>
+__global__ __launch_bounds__(256, NB == 3 && FRAME ? 5 : 4) void sorted_proj_kernel(
+    TorParams p, float4 *rec)
+{
+    const int64_t gid = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
+    record_project<NB, 4, FRAME, true>(p, rec, gid / 4, (int)(gid % 4), gid / 4 < p.n, p.out);
+}
+
+template <bool FRAME>
+int launch_sorted(const TorParams &p, float4 *rec, hipStream_t st)
+{
+    const dim3 grid(blocks_for(4 * p.n, 256)), block(256);
+    switch (p.box) {
+    case 3:
+        hipLaunchKernelGGL((sorted_proj_kernel<3, FRAME>), grid, block, 0, st, p, rec);
+        break;
+    case 4:
+        hipLaunchKernelGGL((sorted_proj_kernel<4, FRAME>), grid, block, 0, st, p, rec);
+        break;
+    default:
+        hipLaunchKernelGGL((sorted_proj_kernel<0, FRAME>), grid, block, 0, st, p, rec);
+        break;
+    }
+    return launch_status();
+}
+
+// Where ordering the events first pays: from 131073 events on (below, lanes
+// that share an event hide the gathers' latency and the four ordering kernels
+// are launch-bound) over images that the gathers of a box walk miss L2 on, or
+// with chord walks, whose patches take more lines.  Events in time order, one
+// lane per event against this path, us: 200 x 200 x 100 x 200k events 298 / 190,
+// x 1M 1165 / 607; 256 x 256 x 160 x 1M 1989 / 798; 181 x 175 x 83 x 400k 380 / 271;
+// 160 x 160 x 80 (8.2 MB) x 400k 213 / 250; chords: 128 x 128 x 64 x 400k 1171 /
+// 650, 181 x 175 x 83 x 1M 4449 / 2112.  Events that come in locality order
+// already, same columns: 197 / 187, 565 / 642, 1112 / 838, 241 / 290, 180 / 258,
+// 763 / 661, 3145 / 2155.
+constexpr int64_t kSortedEvents = 131073;
+constexpr int64_t kSortedBox = 10000000, kSortedChord = 4000000; // bytes of the image
+constexpr int64_t kSortedPiece = (int64_t)1 << 20;               // 151 MB of records
+
+} // namespace
+
+int sorted_project(const TorParams &p, uint32_t flags, hipStream_t st, bool *done)
+{
+    *done = false;
+    constexpr uint32_t sched = (3u << SRFX_LPE_SHIFT) | (3u << SRFX_BLOCK_SHIFT) |
+                               (3u << SRFX_SLAB_SHIFT) | SRFX_FULL_PATCH;
+    const int64_t bytes = (int64_t)4 * p.gx * p.gy * p.gz;
+    if ((flags & sched) || p.n < kSortedEvents ||
+        bytes < (p.box ? kSortedBox : kSortedChord) || !workspace_ok(st))
+        return SRFX_OK;
+    const int64_t piece = std::min<int64_t>(p.n, kSortedPiece);
+    const size_t rb = align256(sizeof(float4) * kWalkF4 * (size_t)piece);
+    char *ws = nullptr;
+    if (ws_alloc((void **)&ws, rb + locality_bytes(piece), st))
+        return SRFX_OK;
+    const bool frame = p.sx == 1 && p.sy == p.gx && p.sz == p.gx * p.gy &&
+                       bytes < ((int64_t)1 << 31) && (int64_t)p.gx * p.gy < ((int64_t)1 << 24);
+    int rc = SRFX_OK;
+    for (int64_t e0 = 0; e0 < p.n && !rc; e0 += piece) {
+        TorParams q = p;
+        q.n = std::min(piece, p.n - e0);
+        q.lors = p.lors + e0;
+        q.out = p.out + e0;
+        q.img_bytes = (int)bytes;
+        LocalityOrder order;
+        rc = locality_order(q, order, ws + rb, st);
+        if (rc)
+            break;
+        hipLaunchKernelGGL(sorted_place_kernel, dim3(blocks_for(q.n, 256)), dim3(256), 0, st, q,
+                           order, (float4 *)ws);
+        rc = frame ? launch_sorted<true>(q, (float4 *)ws, st)
+                   : launch_sorted<false>(q, (float4 *)ws, st);
     }
     *done = true;
     const int rf = ws_free(ws, st);

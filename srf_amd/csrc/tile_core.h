@@ -868,8 +868,9 @@ __device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom
 // the event's backprojection: 1/p for a projection p > 1e-7, else 0 (the
 // event adds nothing, as the reference's ratio skips it), so that each of the
 // event's listings reads it instead of dividing again.  With pout the
-// projection p itself goes to pout[e] instead (the plan's projection op).
-template <int NB, int LPE, bool FRAME = false>
+// projection p itself goes to pout[e] instead (the plan's projection op); SORTED:
+// to pout[i], i the int in the record's value slot.
+template <int NB, int LPE, bool FRAME = false, bool SORTED = false>
 __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, int64_t e,
                                                int sub, bool valid, float *pout = nullptr)
 {
@@ -877,8 +878,11 @@ __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, 
     Event ev;
     Track t;
     bool any = false;
+    int64_t place = e;
     if (valid) {
-        unpack_walk(p, rec, e, ev, t);
+        const float v = unpack_walk(p, rec, e, ev, t);
+        if (SORTED)
+            place = __float_as_int(v);
         any = ev.s_lo <= ev.s_hi;
     }
     // The lanes of a wave walk the same slices at the same time (from the
@@ -889,13 +893,17 @@ __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, 
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1)
         base = min(base, __shfl_xor(base, m, 64));
+    // in an order that differs from call to call, lane sub takes the slices
+    // congruent to it: the same sum whichever events share the wave
+    if (SORTED)
+        base &= ~(LPE - 1);
     if (any)
         part = walk_event<0, NB, FRAME>(p, ev, t, p.use_tof, 0.0f, base + sub, ev.s_hi, LPE,
                                         ev.s_lo);
     const float pv = group_sum<LPE>(part);
     if (valid && sub == 0) {
-        if (pout)
-            pout[e] = pv;
+        if (SORTED || pout)
+            pout[place] = pv;
         else
             reinterpret_cast<float *>(rec)[4 * kWalkHead * e + kWalkValue] =
                 pv > 1e-7 ? 1.0f / pv : 0.0f;

@@ -37,6 +37,10 @@ extern "C" int srfx_tor_project(const float *lors, int64_t n, int64_t ld, const 
     p.img = image;
     p.out = proj;
     hipStream_t st = (hipStream_t)stream;
+    bool done = false;
+    rc = sorted_project(p, flags, st, &done);
+    if (rc || done)
+        return rc;
     int nslab, inter;
     if (!slab_schedule(flags, nslab, inter) || n == 0)
         return launch<kProj>(p, flags, st);
