@@ -11,7 +11,7 @@ autograd_c3  differentiable projector: batch of 8 lumpy 128x128x64 images,
              the memory of recomputation against stored voxel lists.
 batched_c4   64 independent TOF OSEM reconstructions (image sizes mixed from
              96x96x48, 128x128x64, 200x200x100; events log-uniform in
-             [1e5, 5e6]), 2 iterations x 8 subsets: one persistent launch per
+             [1e5, 5e6]), 2 iterations x 8 subsets: one launch per kernel and
              subset replayed from a HIP graph, against the same
              reconstructions run one after another.
 large_c5     256x256x160 (1.6x1.6x1.7 mm) torso phantom, 300M events at

@@ -469,7 +469,8 @@ typedef struct srfx_recon {
 typedef struct srfx_tor_batch srfx_tor_batch;
 
 /* Plan a batch of independent OSEM reconstructions that share one TOR model
- * and one subset count.  Allocates the plan's device tables; no reference
+ * and one subset count.  Allocates the plan's device tables, with the events
+ * in a locality order of the plan's own; no reference
  * counterpart (the reference reconstructs one image per process,
  * graph/reconstruction/local_reconstruction.py:44-51).  SRFX_EUNSUPPORTED for
  * an image of 2^31 bytes or more, or with an op-frame slice of 2^24 voxels or
@@ -479,13 +480,13 @@ int srfx_tor_batch_create(const srfx_recon *recons, int32_t nrecon, int32_t nb_s
 
 /* Advance every reconstruction of the plan by OSEM subset `subset`
  * (ReconStep + mlem_update, model/recon_step.py:33-49, on contiguous subset
- * rows, graph/reconstruction/worker.py:79-85) in one persistent launch.
+ * rows, graph/reconstruction/worker.py:79-85) in one launch per kernel.
  * Enqueues kernels only (no allocation, no memset): capturable in a HIP
  * graph.  Calls on one plan must not overlap. */
 int srfx_tor_batch_subset(srfx_tor_batch *plan, int32_t subset, void *stream);
 
-/* Schedule of the plan's persistent projection: lanes per event (1, 4 or 16)
- * and events per work item a wave pulls (64, 128 or 256); default 4 and 64.
+/* Schedule of the plan's projection: lanes per event (1, 4 or 16)
+ * and events per work item of a wave (64, 128 or 256); default 4 and 64.
  * SRFX_EINVAL for any other pair (the schedule is then unchanged).  Set it
  * before capturing subsets in a HIP graph: a graph keeps the kernel it
  * recorded.  No reference counterpart (launch tuning of the batch). */

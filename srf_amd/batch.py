@@ -4,12 +4,12 @@
 (each a dict with ``image`` (Image), ``emap`` (Image of the inverse efficiency
 map) and ``data`` (ListModeDataSplit from preprocess.recon_process)) that share
 one SplitLoRsModel.  ``run_subset(k)`` advances every reconstruction by OSEM
-subset k (srfx_tor_batch_subset: four kernels, two of them persistent);
+subset k (srfx_tor_batch_subset: five kernels for all reconstructions);
 ``capture()`` records one full iteration (all subsets) into a HIP graph that
 ``replay()`` reruns.  Every (reconstruction, axis group, subset) gets a tile
-plan at creation; a subset step is a persistent projection over the events of
-all reconstructions, a persistent tiled backprojection over the tile chunks of
-all plans and the batched update.  ``serial_iterate`` runs the same
+plan at creation, its events in a locality order; a subset step is a projection
+over the events of all reconstructions, a tiled backprojection over the tile
+chunks of all plans and the batched update.  ``serial_iterate`` runs the same
 reconstructions one after another through the per-reconstruction OSEM driver
 (projection + tiled backprojection), for comparison.
 """
@@ -22,7 +22,7 @@ from .ops import _check_dev, _stream
 from .recon import OSEM
 
 
-# Schedules of the persistent projection: lanes per event x events per work item.
+# Schedules of the projection: lanes per event x events per work item.
 LANES = (1, 4, 16)
 ITEM_EVENTS = (64, 128, 256)
 
@@ -99,7 +99,7 @@ class BatchedOSEM:
         self.schedule = (4, 64)
 
     def set_schedule(self, lanes_per_event, events_per_item):
-        """Schedule of the persistent projection (srfx_tor_batch_set_schedule):
+        """Schedule of the projection (srfx_tor_batch_set_schedule):
         lanes per event in LANES, events per work item in ITEM_EVENTS.  A
         graph keeps the kernel and grid it recorded, so a captured graph is
         dropped: replay() then raises until capture() records the new

@@ -2,24 +2,23 @@
 // and event counts) advance one subset together.
 //
 // At creation every (reconstruction, axis group, subset) gets a tile plan of
-// its events (tile_core.h).  A subset step is four kernels on one stream:
-//   batch_zero     zero every reconstruction's backprojection buffer and the
-//                  work counters (two per box class);
+// its events (tile_core.h), its walk records in a locality order (locality.h)
+// whatever order the events came in.  A subset step is five kernels or so on one
+// stream:
+//   batch_voxels   zero every reconstruction's backprojection buffer;
 //   batch_frames   copy every reconstruction's image into the op frame of
 //                  each of its axis groups (frame_core.h), which the
 //                  projection reads (a box row of voxels shares a line);
-//   batch_project  persistent projection: each block takes the next chunk of
-//                  <= 256 events (of any reconstruction and group) from a
-//                  counter, walks them from their plan's walk records and
+//   batch_project  one wave per item of <= 256 events (of any reconstruction
+//                  and group): walks them from their plan's walk records and
 //                  writes their projections into the records' value slots;
-//   batch_scatter  persistent tiled backprojection of 1/p: each block takes
-//                  the next tile chunk (of any plan), accumulates it in an
-//                  FP64 LDS tile and flushes it into that reconstruction's
-//                  backprojection buffer;
-//   batch_update   x <- x * E * bp for every reconstruction.
-// Every block of a persistent kernel exits once its counter passes the end of
-// the table.  The step allocates nothing and issues no memset, so a caller can
-// capture it in a HIP graph.  Five kernels in all.
+//   batch_scatter  tiled backprojection of 1/p, one workgroup per tile chunk (of
+//                  any plan): accumulates it in an FP64 LDS tile and flushes it
+//                  into that reconstruction's backprojection buffer;
+//   batch_voxels   x <- x * E * bp for every reconstruction.
+// The projection and the scatter are one launch per box class present.  The step
+// allocates nothing and issues no memset, so a caller can capture it in a HIP
+// graph.
 #include <algorithm>
 #include <new>
 #include <vector>
@@ -43,8 +42,8 @@ struct EvChunk {
 };
 
 // Box classes of the batch's jobs: 0 = candidate box 3 with every event on
-// the 3 x 2 box (the single-walk scatter), 1 = other box-3 jobs, 2 = box 4, 3 = chord walk.  Each class has its own work lists
-// and persistent kernels, so that a kernel holds only its class's walk (and
+// the 3 x 2 box (the single-walk scatter), 1 = other box-3 jobs, 2 = box 4, 3 =
+// chord walk.  Each class has its own work lists and kernels, so that a kernel holds only its class's walk (and
 // its registers).
 constexpr int kBoxClasses = 4;
 
@@ -59,116 +58,139 @@ struct TileWork {
     int job, tile, start, count;
 };
 
+// One reconstruction's voxels: workgroups first, first + 1, ... of the
+// elementwise kernels, kVoxBlock voxels each.
 struct VoxRange {
     float *x;
     const float *e;
     float *bp;
     long long n;
-    long long off; // first voxel of this reconstruction in the concatenated range
+    int first;
+    int wide; // the three arrays are 16-byte aligned
 };
 
 namespace {
 
 constexpr int kChunk = 256;
 
-__device__ __forceinline__ int find_range(const VoxRange *r, int nrec, long long i)
+constexpr int kVoxBlock = 4096;
+
+// The reconstruction of workgroup blockIdx.x.
+__device__ __forceinline__ const VoxRange &find_range(const VoxRange *r, int nrec)
 {
     int lo = 0, hi = nrec - 1;
     while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (r[mid].off <= i)
+        const int mid = (lo + hi + 1) >> 1;
+        if (r[mid].first <= (int)blockIdx.x)
             lo = mid;
         else
             hi = mid - 1;
     }
-    return lo;
+    return r[lo];
 }
 
-__global__ __launch_bounds__(256) void batch_zero(const VoxRange *__restrict__ r, int nrec,
-                                                  long long total, unsigned *counters)
+// The elementwise kernels: bound by memory, so one reconstruction per workgroup
+// (the search once, in scalar registers) and 16-byte accesses, four in flight
+// per thread and array.  UPDATE: x <- x * E * bp (model/recon_step.py:48-49),
+// else bp <- 0.  8.9M voxels in 12 reconstructions: update 84 -> 24 us
+// (143 MB), zero 31 -> 7.5, against a grid-stride loop that searched per
+// voxel.
+template <bool UPDATE>
+__global__ __launch_bounds__(256) void batch_voxels(const VoxRange *__restrict__ r, int nrec)
 {
-    if (blockIdx.x == 0 && threadIdx.x < 2 * kBoxClasses)
-        counters[threadIdx.x] = 0u;
-    long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        int k = find_range(r, nrec, i);
-        r[k].bp[i - r[k].off] = 0.0f;
+    const VoxRange &v = find_range(r, nrec);
+    const long long i0 = (long long)((int)blockIdx.x - v.first) * kVoxBlock;
+    float *const x = v.x + i0, *const bp = v.bp + i0;
+    const float *const e = v.e + i0;
+    const int n = (int)min((long long)kVoxBlock, v.n - i0);
+    if (v.wide && n == kVoxBlock) {
+        constexpr int N = kVoxBlock / 1024;
+        float4 fx[N], fe[N], fb[N];
+        if (UPDATE) {
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                fx[k] = reinterpret_cast<const float4 *>(x)[k * 256 + threadIdx.x];
+                fe[k] = reinterpret_cast<const float4 *>(e)[k * 256 + threadIdx.x];
+                fb[k] = reinterpret_cast<const float4 *>(bp)[k * 256 + threadIdx.x];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            if (UPDATE)
+                reinterpret_cast<float4 *>(x)[k * 256 + threadIdx.x] =
+                    make_float4((fx[k].x * fe[k].x) * fb[k].x, (fx[k].y * fe[k].y) * fb[k].y,
+                                (fx[k].z * fe[k].z) * fb[k].z, (fx[k].w * fe[k].w) * fb[k].w);
+            else
+                reinterpret_cast<float4 *>(bp)[k * 256 + threadIdx.x] =
+                    make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i < n; i += 256) {
+        if (UPDATE)
+            x[i] = (x[i] * e[i]) * bp[i];
+        else
+            bp[i] = 0.0f;
     }
 }
 
-// model/recon_step.py:48-49 for every reconstruction.
-__global__ __launch_bounds__(256) void batch_update(const VoxRange *__restrict__ r, int nrec,
-                                                    long long total)
+// Item of workgroup blockIdx.x (xcd_groups's grid): workgroup b runs on XCD
+// b % 8, and each XCD takes runs of g neighbouring items, so that its L2 serves
+// one part of one reconstruction's frame at a time while the XCDs stay level.
+__device__ __forceinline__ int xcd_item(int g)
 {
-    long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        int k = find_range(r, nrec, i);
-        long long j = i - r[k].off;
-        r[k].x[j] = (r[k].x[j] * r[k].e[j]) * r[k].bp[j];
-    }
+    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
+    return (i / g * 8 + x) * g + i % g;
 }
 
-// Next work item of a persistent wave (the same value in every lane; every
-// lane active).
-__device__ __forceinline__ int next_wave_item(unsigned *counter)
-{
-    int item = 0;
-    if (__lane_id() == 0)
-        item = (int)atomicAdd(counter, 1u);
-    return __builtin_amdgcn_readfirstlane(item);
-}
-
-// Waves pull work items of T events from the event chunks (kChunk / T items
-// per chunk) of one box class (NB), walked in rounds of 64 / LPE events at
-// LPE lanes per event, without synchronising with the other waves of their
-// block, so a wave with long walks holds up no other.  The default schedule,
+// One wave per work item of T events (kChunk / T items per event chunk) of one
+// box class (NB), walked in rounds of 64 / LPE events at LPE lanes per event.
+// The hardware deals the waves out: pulling items from a counter in memory takes
+// about 20 ns a pull whoever asks, 9300 items and 5120 waves that find it empty
+// here.  594k events in 12 reconstructions (128 x 128 x 64), one lane per event:
+// 340 us from a counter in the order the events came, 304 in locality order, 242
+// dealt out by the hardware, 229 with the runs of xcd_item short enough that an
+// XCD's waves share a frame's part (four lanes: 217).  The default schedule,
 // LPE = 4 and T = 64 (quarter chunks), is the projection schedule of the plan
 // OSEM step.  The gathers read the jobs' contiguous op frames
-// (record_project<.., true>).  Five waves per SIMD for the 3 x 3 box at one
-// lane per event and items of up to 128 events (a 12-byte spill outside the
-// walk; C4 iteration 88 against 93 ms); the other schedules measured slower
-// at five and keep four.
+// (record_project<.., true>).  Five waves per SIMD for the 3 x 3 box at up to four
+// lanes per event and items of up to 128 events (four lanes: 235 against 260 us at
+// four waves); the other schedules measured slower at five and keep four.
 template <int NB, int LPE, int T>
-__global__ __launch_bounds__(256, NB == 3 && LPE == 1 && T <= 128 ? 5 : 4) void batch_project(
-    const BatchJob *__restrict__ jobs, const EvChunk *__restrict__ chunks, int nchunks,
-    unsigned *counter)
+__global__ __launch_bounds__(64, NB == 3 && LPE <= 4 && T <= 128 ? 5 : 4) void batch_project(
+    const BatchJob *__restrict__ jobs, const EvChunk *__restrict__ chunks, int nchunks, int group)
 {
     constexpr int kParts = kChunk / T, kRound = 64 / LPE;
     static_assert(kChunk % T == 0 && T % kRound == 0, "items split chunks into whole rounds");
-    for (;;) {
-        const int q = next_wave_item(counter);
-        if (q >= kParts * nchunks)
-            break;
-        const EvChunk ch = chunks[q / kParts];
-        const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(ch.job)];
-        float4 *rec = const_cast<float4 *>(job.rec);
-        const int lane = (int)__lane_id(), sub = lane % LPE;
-        for (int r = 0; r < T; r += kRound) {
-            const int i = (q % kParts) * T + r + lane / LPE;
-            const bool valid = i < ch.count;
-            const int64_t e = (int64_t)ch.start + i;
-            record_project<NB, LPE, true>(job.p, rec, e, sub, valid);
-        }
+    const int q = xcd_item(group);
+    if (q >= kParts * nchunks)
+        return;
+    const EvChunk ch = chunks[q / kParts];
+    const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(ch.job)];
+    float4 *rec = const_cast<float4 *>(job.rec);
+    const int lane = (int)__lane_id(), sub = lane % LPE;
+    for (int r = 0; r < T; r += kRound) {
+        const int i = (q % kParts) * T + r + lane / LPE;
+        const bool valid = i < ch.count;
+        const int64_t e = (int64_t)ch.start + i;
+        record_project<NB, LPE, true>(job.p, rec, e, sub, valid);
     }
 }
 
-// Blocks pull tile chunks of one box class (NB); four waves per SIMD where
+// One workgroup per tile chunk of one box class (NB); four waves per SIMD where
 // the walk fits, five for the single-walk class (ONE), as tile_scatter.
 template <int NB, bool ONE = false>
 __global__ __launch_bounds__(256, ONE ? 5 : (NB == 4 ? 3 : 4)) void batch_scatter(
-    const BatchJob *__restrict__ jobs, const TileWork *__restrict__ work, int nwork,
-    unsigned *counter)
+    const BatchJob *__restrict__ jobs, const TileWork *__restrict__ work, int nwork, int group)
 {
     extern __shared__ double ldsd[];
-    for (;;) {
-        const int c = next_item(counter);
-        if (c >= nwork)
-            break;
-        const TileWork w = work[c];
-        const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(w.job)];
-        const TileChunk ch{w.tile, w.start, w.count, 0};
-        scatter_chunk<kBack, NB, true, ONE>(job.p, job.g, ch, job.list, job.rec, ldsd);
-    }
+    const int c = xcd_item(group);
+    if (c >= nwork)
+        return;
+    const TileWork w = work[c];
+    const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(w.job)];
+    const TileChunk ch{w.tile, w.start, w.count, 0};
+    scatter_chunk<kBack, NB, true, ONE>(job.p, job.g, ch, job.list, job.rec, ldsd);
 }
 
 // One op-frame copy: the world image read with the group's op-frame strides
@@ -238,8 +260,7 @@ struct srfx_tor_batch {
     std::vector<srfx::TileWork *> d_work;
     std::vector<int> nwork;
     srfx::VoxRange *d_vox = nullptr;
-    long long total_vox = 0;
-    unsigned *d_counters = nullptr;
+    unsigned vox_blocks = 0;
     // the block holding the op-frame copies, one per (reconstruction,
     // non-empty group)
     std::vector<float *> frames;
@@ -247,49 +268,52 @@ struct srfx_tor_batch {
     int nframes = 0;
     long long frame_blocks = 0;
     unsigned scatter_lds = 0;
-    int proj_blocks[srfx::kBoxClasses] = {}, scatter_blocks[srfx::kBoxClasses] = {};
-    int elem_blocks = 0;
     int cus = 0;
     int proj_lanes = 4, proj_events = 64; // projection schedule (batch_project<LPE, T>)
 };
 
 using namespace srfx;
 
-// The persistent projection of schedule (LPE, T): with subset < 0 sets the
-// plan's grid from the kernel's occupancy, else enqueues it for that subset.
-template <int NB, int LPE, int T>
-static int project_class(srfx_tor_batch *b, int c, int subset, hipStream_t st)
+// Grid and run length of xcd_item for n items: runs of at most `room` (for the
+// projection a fifth of the waves an XCD holds: 4 to 16 waves per CU measured
+// 229 / 242 us, contiguous eighths 255; for the scatter one workgroup per CU, 155
+// against 159 to 271).
+static unsigned xcd_groups(int64_t n, int room, int &group)
 {
-    if (subset < 0) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_project<NB, LPE, T>, 256,
-                                                         0) != hipSuccess)
-            return SRFX_ELAUNCH;
-        b->proj_blocks[c] = std::max(1, b->cus * std::max(1, per_cu));
-        return SRFX_OK;
-    }
+    const int64_t k = std::max<int64_t>(1, (n + 8 * room - 1) / (8 * room));
+    group = (int)std::max<int64_t>(1, (n + 8 * k - 1) / (8 * k));
+    return (unsigned)(8 * k * group);
+}
+
+// Enqueue the projection of one box class with schedule (LPE, T) for a subset.
+template <int NB, int LPE, int T>
+static void project_class(const srfx_tor_batch *b, int c, int subset, hipStream_t st)
+{
     const int w = subset * kBoxClasses + c;
-    if (b->nev[w] > 0)
-        hipLaunchKernelGGL((batch_project<NB, LPE, T>), dim3(b->proj_blocks[c]), dim3(256), 0, st,
-                           b->d_jobs, b->d_ev[w], b->nev[w], b->d_counters + 2 * c);
-    return SRFX_OK;
+    if (b->nev[w] == 0)
+        return;
+    int group;
+    const unsigned grid = xcd_groups((int64_t)(kChunk / T) * b->nev[w], 4 * b->cus / 8, group);
+    hipLaunchKernelGGL((batch_project<NB, LPE, T>), dim3(grid), dim3(64), 0, st, b->d_jobs,
+                       b->d_ev[w], b->nev[w], group);
 }
 
 template <int LPE, int T>
-static int project_launch(srfx_tor_batch *b, int subset, hipStream_t st)
+static int project_launch(const srfx_tor_batch *b, int subset, hipStream_t st)
 {
-    int rc = project_class<3, LPE, T>(b, 0, subset, st);
-    if (!rc)
-        rc = project_class<3, LPE, T>(b, 1, subset, st);
-    if (!rc)
-        rc = project_class<4, LPE, T>(b, 2, subset, st);
-    if (!rc)
-        rc = project_class<0, LPE, T>(b, 3, subset, st);
-    return rc;
+    if (subset < 0)
+        return SRFX_OK;
+    project_class<3, LPE, T>(b, 0, subset, st);
+    project_class<3, LPE, T>(b, 1, subset, st);
+    project_class<4, LPE, T>(b, 2, subset, st);
+    project_class<0, LPE, T>(b, 3, subset, st);
+    return SRFX_OK;
 }
 
-// Lanes per event {1, 4, 16} x events per work item {64, 128, 256}.
-static int project_schedule(srfx_tor_batch *b, int lanes, int events, int subset, hipStream_t st)
+// Lanes per event {1, 4, 16} x events per work item {64, 128, 256}; subset < 0
+// only checks the schedule.
+static int project_schedule(const srfx_tor_batch *b, int lanes, int events, int subset,
+                            hipStream_t st)
 {
     if (lanes == 1 && events == 64)
         return project_launch<1, 64>(b, subset, st);
@@ -325,7 +349,6 @@ static void free_plan(srfx_tor_batch *b)
     for (TileWork *w : b->d_work)
         (void)hipFree(w);
     (void)hipFree(b->d_vox);
-    (void)hipFree(b->d_counters);
     for (float *f : b->frames)
         (void)hipFree(f);
     (void)hipFree(b->d_frames);
@@ -376,7 +399,7 @@ extern "C" int srfx_tor_batch_create(const srfx_recon *recons, int32_t nrecon,
     std::vector<std::vector<TileWork>> work((size_t)nb_subsets * kBoxClasses);
     std::vector<VoxRange> vox;
     std::vector<FrameJob> frames;
-    long long off = 0;
+    long long vox_blocks = 0;
     int rc_status = SRFX_OK;
     // one block for the op-frame copies of every (reconstruction, non-empty
     // group), carved in the loop below
@@ -407,7 +430,7 @@ extern "C" int srfx_tor_batch_create(const srfx_recon *recons, int32_t nrecon,
             for (int k = 0; k <= nb_subsets; k++)
                 bd[k] = k * rc.n[a] / nb_subsets;
             requests.push_back(SubsetRequest{rc.lors[a], rc.n[a], rc.ld[a], group_grid(rc, a),
-                                             kBatchTile, nb_subsets, bd.data()});
+                                             kBatchTile, nb_subsets, bd.data(), true});
         }
     std::vector<srfx_tor_plan> all_plans(requests.size() * nb_subsets, nullptr);
     rc_status = plan_create_subsets_many(requests.data(), (int)requests.size(), 10, m,
@@ -485,21 +508,27 @@ extern "C" int srfx_tor_batch_create(const srfx_recon *recons, int32_t nrecon,
             }
         }
         long long nv = (long long)rc.shape[0] * rc.shape[1] * rc.shape[2];
-        vox.push_back(VoxRange{rc.image, rc.emap, rc.bp, nv, off});
-        off += nv;
+        const uintptr_t at = (uintptr_t)rc.image | (uintptr_t)rc.emap | (uintptr_t)rc.bp;
+        vox.push_back(VoxRange{rc.image, rc.emap, rc.bp, nv, (int)vox_blocks, at % 16 == 0});
+        vox_blocks += (nv + kVoxBlock - 1) / kVoxBlock;
     }
     if (rc_status) {
         free_plan(b);
         return rc_status;
     }
     b->njobs = (int)jobs.size();
-    b->total_vox = off;
+    b->vox_blocks = (unsigned)vox_blocks;
     b->nframes = (int)frames.size();
-    bool ok = upload(&b->d_jobs, jobs) && upload(&b->d_vox, vox) && upload(&b->d_frames, frames) &&
-              hipMalloc(&b->d_counters, 2 * kBoxClasses * sizeof(unsigned)) == hipSuccess;
+    bool ok = upload(&b->d_jobs, jobs) && upload(&b->d_vox, vox) && upload(&b->d_frames, frames);
     for (size_t w = 0; ok && w < ev.size(); w++) {
         EvChunk *e = nullptr;
         TileWork *t = nullptr;
+        // The longest chunks first, so that the last workgroups to run are short
+        // (5100 chunks on 1280 places: 180 us in plan order, 155 so); by 256 events,
+        // to keep neighbours together.
+        std::stable_sort(work[w].begin(), work[w].end(), [](const TileWork &a, const TileWork &b) {
+            return a.count / 256 > b.count / 256;
+        });
         ok = upload(&e, ev[w]) && upload(&t, work[w]);
         b->d_ev.push_back(e);
         b->nev.push_back((int)ev[w].size());
@@ -507,26 +536,14 @@ extern "C" int srfx_tor_batch_create(const srfx_recon *recons, int32_t nrecon,
         b->nwork.push_back((int)work[w].size());
     }
     b->scatter_lds = (unsigned)(sizeof(double) * kBatchTile.slices * kBatchTile.wx * kBatchTile.wy);
-    int dev = 0, cus = 0, per_cu_s[kBoxClasses] = {};
+    int dev = 0, cus = 0;
     ok = ok && hipGetDevice(&dev) == hipSuccess &&
-         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_s[0], batch_scatter<3, true>, 256,
-                                                      b->scatter_lds) == hipSuccess &&
-         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_s[1], batch_scatter<3>, 256,
-                                                      b->scatter_lds) == hipSuccess &&
-         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_s[2], batch_scatter<4>, 256,
-                                                      b->scatter_lds) == hipSuccess &&
-         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_s[3], batch_scatter<0>, 256,
-                                                      b->scatter_lds) == hipSuccess;
-    b->cus = cus;
-    ok = ok && project_schedule(b, b->proj_lanes, b->proj_events, -1, nullptr) == SRFX_OK;
+         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
     if (!ok) {
         free_plan(b);
         return SRFX_ELAUNCH;
     }
-    for (int c = 0; c < kBoxClasses; c++)
-        b->scatter_blocks[c] = std::max(1, cus * std::max(1, per_cu_s[c]));
-    b->elem_blocks = std::max(1, cus * 4);
+    b->cus = cus;
     *out = b;
     return SRFX_OK;
 }
@@ -536,8 +553,8 @@ extern "C" int srfx_tor_batch_subset(srfx_tor_batch *b, int32_t subset, void *st
     if (!b || subset < 0 || subset >= b->nsub)
         return SRFX_EINVAL;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(batch_zero, dim3(b->elem_blocks), dim3(256), 0, st, b->d_vox, b->nrec,
-                       b->total_vox, b->d_counters);
+    hipLaunchKernelGGL(batch_voxels<false>, dim3(b->vox_blocks), dim3(256), 0, st, b->d_vox,
+                       b->nrec);
     if (b->nframes > 0)
         hipLaunchKernelGGL(batch_frames, dim3((unsigned)b->frame_blocks), dim3(256), 0, st,
                            b->d_frames, b->nframes);
@@ -546,25 +563,17 @@ extern "C" int srfx_tor_batch_subset(srfx_tor_batch *b, int32_t subset, void *st
         const int w = subset * kBoxClasses + c;
         if (b->nwork[w] == 0)
             continue;
-        if (c == 0)
-            hipLaunchKernelGGL((batch_scatter<3, true>), dim3(b->scatter_blocks[c]), dim3(256),
-                               b->scatter_lds, st, b->d_jobs, b->d_work[w], b->nwork[w],
-                               b->d_counters + 2 * c + 1);
-        else if (c == 1)
-            hipLaunchKernelGGL(batch_scatter<3>, dim3(b->scatter_blocks[c]), dim3(256),
-                               b->scatter_lds, st, b->d_jobs, b->d_work[w], b->nwork[w],
-                               b->d_counters + 2 * c + 1);
-        else if (c == 2)
-            hipLaunchKernelGGL(batch_scatter<4>, dim3(b->scatter_blocks[c]), dim3(256),
-                               b->scatter_lds, st, b->d_jobs, b->d_work[w], b->nwork[w],
-                               b->d_counters + 2 * c + 1);
-        else
-            hipLaunchKernelGGL(batch_scatter<0>, dim3(b->scatter_blocks[c]), dim3(256),
-                               b->scatter_lds, st, b->d_jobs, b->d_work[w], b->nwork[w],
-                               b->d_counters + 2 * c + 1);
+        int group;
+        const dim3 grid(xcd_groups(b->nwork[w], b->cus / 8, group)), block(256);
+        auto *kernel = c == 0   ? batch_scatter<3, true>
+                       : c == 1 ? batch_scatter<3>
+                       : c == 2 ? batch_scatter<4>
+                                : batch_scatter<0>;
+        hipLaunchKernelGGL(kernel, grid, block, b->scatter_lds, st, b->d_jobs, b->d_work[w],
+                           b->nwork[w], group);
     }
-    hipLaunchKernelGGL(batch_update, dim3(b->elem_blocks), dim3(256), 0, st, b->d_vox, b->nrec,
-                       b->total_vox);
+    hipLaunchKernelGGL(batch_voxels<true>, dim3(b->vox_blocks), dim3(256), 0, st, b->d_vox,
+                       b->nrec);
     return launch_status();
 }
 

@@ -436,7 +436,7 @@ int sorted_project(const TorParams &p, uint32_t flags, hipStream_t st, bool *don
     const int64_t piece = std::min<int64_t>(p.n, kSortedPiece);
     const size_t rb = align256(sizeof(float4) * kWalkF4 * (size_t)piece);
     char *ws = nullptr;
-    if (ws_alloc((void **)&ws, rb + locality_bytes(piece), st))
+    if (ws_alloc((void **)&ws, rb + locality_bytes(piece, 1), st))
         return SRFX_OK;
     const bool frame = p.sx == 1 && p.sy == p.gx && p.sz == p.gx * p.gy &&
                        bytes < ((int64_t)1 << 31) && (int64_t)p.gx * p.gy < ((int64_t)1 << 24);
@@ -448,7 +448,7 @@ int sorted_project(const TorParams &p, uint32_t flags, hipStream_t st, bool *don
         q.out = p.out + e0;
         q.img_bytes = (int)bytes;
         LocalityOrder order;
-        rc = locality_order(q, order, ws + rb, st);
+        rc = locality_order(q, 1, order, ws + rb, st);
         if (rc)
             break;
         hipLaunchKernelGGL(sorted_place_kernel, dim3(blocks_for(q.n, 256)), dim3(256), 0, st, q,

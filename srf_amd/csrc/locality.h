@@ -8,16 +8,20 @@ namespace srfx {
 // The buckets of a set's events and each bucket's next free place: a kernel
 // over the events puts event e at place atomicAdd(&cursor[key[e]], 1), where
 // neighbouring places hold near and nearly parallel tubes (order within a
-// bucket arbitrary).
+// bucket arbitrary), subset [k n / K, (k + 1) n / K) to places of that range.
 struct LocalityOrder {
     const int *key;
     unsigned *cursor;
 };
 
-// Workspace bytes of locality_order for n events.
-size_t locality_bytes(int64_t n);
+// Workspace bytes of the order of n events in K subsets.
+size_t locality_bytes(int64_t n, int64_t K);
 
-// The order of the events of p, in the workspace ws of locality_bytes(p.n).
-int locality_order(const TorParams &p, LocalityOrder &order, char *ws, hipStream_t st);
+// The order of the events of p in K subsets, in the workspace ws of
+// locality_bytes(p.n, K).
+int locality_order(const TorParams &p, int64_t K, LocalityOrder &order, char *ws, hipStream_t st);
+
+// place[e] = the place of event e.
+int locality_places(const TorParams &p, int64_t K, int *place, char *ws, hipStream_t st);
 
 } // namespace srfx

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kRangeBlocks) void locality_bits(const float *__res
 }
 
 // Bucket of every event and the buckets' counts.
-__global__ __launch_bounds__(256) void locality_count(TorParams p, int bits,
+__global__ __launch_bounds__(256) void locality_count(TorParams p, int64_t K, int bits,
                                                       const LocalityState *s, int *key,
                                                       unsigned *hist)
 {
@@ -197,6 +197,15 @@ __global__ __launch_bounds__(256) void locality_count(TorParams p, int bits,
         const int x = d == 0 ? v[0] : (d == 1 ? v[1] : (d == 2 ? v[2] : (d == 3 ? v[3] : v[4])));
         k = 2 * k + ((x >> (sq >> 8)) & 1);
     }
+    int64_t sub = 0;
+    if (K > 1) { // the subset with sub n / K <= e < (sub + 1) n / K
+        sub = e * K / p.n;
+        while (sub + 1 < K && (sub + 1) * p.n / K <= e)
+            sub++;
+        while (sub > 0 && sub * p.n / K > e)
+            sub--;
+    }
+    k |= (int)(sub << bits);
     key[e] = k;
     atomicAdd(&hist[k], 1u);
 }
@@ -219,27 +228,37 @@ __global__ __launch_bounds__(kScan) void locality_scan(const unsigned *__restric
         first[i] = (unsigned)(base + o);
 }
 
-// Key bits: about eight events a bucket.
-int key_bits(int64_t n)
+__global__ __launch_bounds__(256) void locality_place(int64_t n, LocalityOrder o, int *place)
 {
-    int b = 4;
-    while (b < kMaxBits && (int64_t)8 << (b + 1) <= n)
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < n)
+        place[e] = (int)atomicAdd(&o.cursor[o.key[e]], 1u);
+}
+
+// Key bits of a subset: about eight events a bucket, at most 2^16 buckets in all
+// unless the subsets alone take more.
+int key_bits(int64_t n, int64_t K)
+{
+    int b = 0;
+    while (b < kMaxBits && (K << (b + 1)) <= ((int64_t)1 << kMaxBits) &&
+           (K << (b + 4)) <= n)
         b++;
     return b;
 }
 
 } // namespace
 
-size_t locality_bytes(int64_t n)
+size_t locality_bytes(int64_t n, int64_t K)
 {
     return align256(sizeof(LocalityState)) + align256(sizeof(float) * 2 * kDims * kRangeBlocks) +
-           2 * align256(sizeof(unsigned) << key_bits(n)) + align256(sizeof(int) * (size_t)n);
+           2 * align256(sizeof(unsigned) * (size_t)(K << key_bits(n, K))) +
+           align256(sizeof(int) * (size_t)n);
 }
 
-int locality_order(const TorParams &p, LocalityOrder &order, char *ws, hipStream_t st)
+int locality_order(const TorParams &p, int64_t K, LocalityOrder &order, char *ws, hipStream_t st)
 {
-    const int bits = key_bits(p.n);
-    const int64_t nh = (int64_t)1 << bits;
+    const int bits = key_bits(p.n, K);
+    const int64_t nh = K << bits;
     auto *s = (LocalityState *)ws;
     auto *part = (float *)(ws + align256(sizeof(LocalityState)));
     auto *hist = (unsigned *)((char *)part + align256(sizeof(float) * 2 * kDims * kRangeBlocks));
@@ -249,10 +268,20 @@ int locality_order(const TorParams &p, LocalityOrder &order, char *ws, hipStream
     const int parts = (int)std::min(eb.x, (unsigned)kRangeBlocks);
     hipLaunchKernelGGL(locality_range, dim3(parts), b, 0, st, p, part, hist, nh);
     hipLaunchKernelGGL(locality_bits, dim3(1), dim3(kRangeBlocks), 0, st, part, parts, s, bits);
-    hipLaunchKernelGGL(locality_count, eb, b, 0, st, p, bits, s, key, hist);
+    hipLaunchKernelGGL(locality_count, eb, b, 0, st, p, K, bits, s, key, hist);
     hipLaunchKernelGGL(locality_scan, dim3((unsigned)((nh + kScan - 1) / kScan)), dim3(kScan), 0,
                        st, hist, first, nh);
     order = LocalityOrder{key, first};
+    return launch_status();
+}
+
+int locality_places(const TorParams &p, int64_t K, int *place, char *ws, hipStream_t st)
+{
+    LocalityOrder o;
+    const int rc = locality_order(p, K, o, ws, st);
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(locality_place, dim3(blocks_for(p.n, 256)), dim3(256), 0, st, p.n, o, place);
     return launch_status();
 }
 

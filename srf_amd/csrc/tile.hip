@@ -5,6 +5,7 @@
 #include <cstring>
 #include <vector>
 
+#include "locality.h"
 #include "tile_core.h"
 
 using namespace srfx;
@@ -299,6 +300,7 @@ struct PlanSet {
     const int64_t *first; // K + 1
     const float *lors;
     int chunk;
+    bool locality = false;
 };
 
 // Build every set of `sets` in shared phases: the count passes of all sets,
@@ -358,7 +360,20 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
     // NB x (NB - 1) box, the chunk sort's jobs
     const size_t ctr_b = align256(sizeof(int) * std::max<size_t>(ctr_n, 1));
     const size_t sjobs_at = align256(head_b + ctr_b + sizeof(int) * (S + nplans));
-    const size_t tmp_b = sjobs_at + sizeof(SortJob) * nplans;
+    // and the places of the events of the sets in locality order with the largest
+    // of their workspaces
+    const size_t place_at = align256(sjobs_at + sizeof(SortJob) * nplans);
+    std::vector<size_t> place_off(S, 0);
+    size_t place_end = place_at, order_b = 0;
+    for (int s = 0; s < S; s++) {
+        const int64_t n = sets[s].first[sets[s].K];
+        if (!sets[s].locality || n <= 0 || n > INT32_MAX)
+            continue;
+        place_off[s] = place_end;
+        place_end += align256(sizeof(int) * (size_t)n);
+        order_b = std::max(order_b, locality_bytes(n, sets[s].K));
+    }
+    const size_t tmp_b = place_end + order_b;
     char *tmp = nullptr, *blk0 = nullptr, *blk1 = nullptr;
     std::vector<char> head(head_b);
     std::vector<int> ctr(ctr_n);
@@ -382,6 +397,7 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
         a.lds = 3u * sizeof(int) * l.nt <= 65536u;
         a.queue = fill_queue_entries(l.nt);
         a.first = (const int64_t *)(tmp + l.head);
+        a.place = place_off[s] ? (const int *)(tmp + place_off[s]) : nullptr;
         a.rec = (float4 *const *)(tmp + l.head + sizeof(int64_t) * (ps.K + 1));
         a.list = (int *const *)(tmp + l.head + sizeof(int64_t) * (ps.K + 1) +
                                 sizeof(void *) * ps.K);
@@ -403,6 +419,14 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
             p.lors = ps.lors;
             const unsigned lds = (a.lds ? (fill ? 3u : 1u) * sizeof(int) * L[s].nt : 0u) +
                                  (fill && a.queue ? fill_queue_lds(a.queue) : 0u);
+            if (!fill && a.place) {
+                TorParams q = p;
+                q.n = n;
+                const int ro = locality_places(q, ps.K, (int *)(tmp + place_off[s]),
+                                               tmp + place_end, st);
+                if (ro)
+                    return ro;
+            }
             if (fill)
                 hipLaunchKernelGGL(plan_set_pass<true>, dim3(blocks_for(n, 256)), dim3(256), lds,
                                    st, p, L[s].g, a);
@@ -803,7 +827,7 @@ int plan_create_subsets_many(const SubsetRequest *req, int nreq, int32_t ncols,
             for (int r = 0, i = 0; r < nreq; i += req[r].nplans, r++)
                 sets.push_back(PlanSet{pls.data() + i, req[r].nplans, first[r].data(),
                                        req[r].lors ? req[r].lors + req[r].bounds[0] : nullptr,
-                                       req[r].tile.chunk});
+                                       req[r].tile.chunk, req[r].locality});
             rc = plan_build_sets(sets, st);
         } else {
             for (int r = 0, i = 0; r < nreq && !rc; r++)

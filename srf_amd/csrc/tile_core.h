@@ -387,6 +387,8 @@ struct PlanSetArgs {
     int queue;              // fill pass: LDS also holds listing queues of this many
                             // entries per wave (0: no queues)
     const int64_t *first;   // [nplans + 1]
+    const int *place;       // count pass: the set's place of each event's record, or null
+                            // (in order); the fill pass follows the records
     float4 *const *rec;     // [nplans] walk records
     int *cnt;               // count pass: listings per (plan, tile); fill pass: read
     const int *off;         // fill pass: first slot of each (plan, tile) in the plan's list
@@ -526,7 +528,7 @@ __global__ __launch_bounds__(256) void plan_set_pass(TorParams p, TileGeom g, Pl
             ok = plan_init(q, a.cols7, r, eg, ev);
             if (ok)
                 make_track(q, ev, eg, r, t);
-            pack_walk(q, r, ev, t, ok, a.rec[k], le);
+            pack_walk(q, r, ev, t, ok, a.rec[k], a.place ? a.place[e] - a.first[k] : le);
             if (ok && q.box > 0 && !shape_one(q, t))
                 flag_other(&a.other[k]);
         }
@@ -1211,6 +1213,9 @@ struct SubsetRequest {
     srfx_tile tile;
     int32_t nplans;
     const int64_t *bounds;
+    // records (and the events' numbers in the plan) in a locality order; needs
+    // bounds k n / nplans
+    bool locality = false;
 };
 int plan_create_subsets_many(const SubsetRequest *req, int nreq, int32_t ncols,
                              const srfx_tor_model &m, srfx_tor_plan *plans, hipStream_t st);
