@@ -168,9 +168,9 @@ __global__ __launch_bounds__(64, NB == 3 && LPE <= 4 && T <= 128 ? 5 : 4) void b
     const EvChunk ch = chunks[q / kParts];
     const BatchJob &job = jobs[__builtin_amdgcn_readfirstlane(ch.job)];
     float4 *rec = const_cast<float4 *>(job.rec);
-    const int lane = (int)__lane_id(), sub = lane % LPE;
+    const int lane = (int)__lane_id(), sub = lane / kRound;
     for (int r = 0; r < T; r += kRound) {
-        const int i = (q % kParts) * T + r + lane / LPE;
+        const int i = (q % kParts) * T + r + lane % kRound;
         const bool valid = i < ch.count;
         const int64_t e = (int64_t)ch.start + i;
         record_project<NB, LPE, true>(job.p, rec, e, sub, valid);

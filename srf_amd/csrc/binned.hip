@@ -387,7 +387,8 @@ __global__ __launch_bounds__(256, NB == 3 && FRAME ? 5 : 4) void sorted_proj_ker
     TorParams p, float4 *rec)
 {
     const int64_t gid = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
-    record_project<NB, 4, FRAME, true>(p, rec, gid / 4, (int)(gid % 4), gid / 4 < p.n, p.out);
+    const int64_t e = gid / 64 * 16 + (int)(gid % 16);
+    record_project<NB, 4, FRAME, true>(p, rec, e, (int)(gid % 64) / 16, e < p.n, p.out);
 }
 
 template <bool FRAME>

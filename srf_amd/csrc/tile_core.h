@@ -872,6 +872,9 @@ __device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom
 // event's listings reads it instead of dividing again.  With pout the
 // projection p itself goes to pout[e] instead (the plan's projection op); SORTED:
 // to pout[i], i the int in the record's value slot.
+// The lanes of an event are 64 / LPE apart: neighbouring lanes are neighbouring
+// events on the same slice, whose loads share lines (side by side on different
+// slices they never do; 8M events, one iteration, 6430 -> 6345 us).
 template <int NB, int LPE, bool FRAME = false, bool SORTED = false>
 __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, int64_t e,
                                                int sub, bool valid, float *pout = nullptr)
@@ -902,7 +905,10 @@ __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, 
     if (any)
         part = walk_event<0, NB, FRAME>(p, ev, t, p.use_tof, 0.0f, base + sub, ev.s_hi, LPE,
                                         ev.s_lo);
-    const float pv = group_sum<LPE>(part);
+    float pv = part;
+#pragma unroll
+    for (int m = 64 / LPE; m < 64; m <<= 1)
+        pv += __shfl_xor(pv, m, 64);
     if (valid && sub == 0) {
         if (SORTED || pout)
             pout[place] = pv;
@@ -932,8 +938,8 @@ __global__ __launch_bounds__(256, NB == 3 && FRAME && LPE <= 4 ? 5 : 4) void rec
     TorParams p, float4 *rec, float *pout)
 {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t e = gid / LPE;
-    record_project<NB, LPE, FRAME>(p, rec, e, (int)(gid % LPE), e < p.n, pout);
+    const int64_t e = gid / 64 * (64 / LPE) + (int)(gid % (64 / LPE));
+    record_project<NB, LPE, FRAME>(p, rec, e, (int)(gid % 64) / (64 / LPE), e < p.n, pout);
 }
 
 
