@@ -119,7 +119,8 @@ __global__ __launch_bounds__(256) void bin_sort(BinTables b)
 }
 
 // tile_scatter over the device's chunk table: workgroups pull chunks.  Both
-// forms are launched; the one whose walk does not fit the events returns.
+// forms are launched; the one whose walk does not fit the events returns.  The
+// scale stays out of the weights' exponent, as in the direct scatter.
 template <int MODE, int NB, bool VREC, bool ONE>
 __global__ __launch_bounds__(256, NB == 4 ? (ONE ? 4 : 3) : (ONE ? 5 : 4)) void bin_scatter(
     TorParams p, TileGeom g, BinTables b)
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(256, NB == 4 ? (ONE ? 4 : 3) : (ONE ? 5 : 4)) void 
         const int c = next_item(&b.state->next[ONE ? 0 : 1]);
         if (c >= n)
             break;
-        scatter_chunk<MODE, NB, VREC, ONE>(p, g, b.chunks[c], b.list0, b.rec0, ldsd);
+        scatter_chunk<MODE, NB, VREC, ONE, false>(p, g, b.chunks[c], b.list0, b.rec0, ldsd);
     }
 }
 

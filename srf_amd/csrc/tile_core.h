@@ -711,10 +711,11 @@ __device__ __forceinline__ float window_walk(const TorParams &p, const TileGeom 
 //     (lo, hi) on its first column / row, so the offsets need no integer
 //     round trip; clipped candidates get an infinite term (neither kept nor
 //     near).
-//   * The scale, the TOF constant and the slice's TOF factor folded into each
-//     kept candidate's exponent, exp2(cw dt + thr cw + log2 |scale tofk| +
-//     TOF quadratic), times the sign of the scale unless POS (a positive
-//     scale: the ratio backprojection).
+//   * The slice's TOF factor folded into each kept candidate's exponent,
+//     exp2(cw dt + thr cw + TOF quadratic), with POS (a positive scale: the
+//     ratio backprojection) log2(scale tofk) as well; else scale tofk is a
+//     factor of its own, so that a scale far from 1 costs the exponent no
+//     digits.
 //   * LDS byte offsets carried from slice to slice.
 // The same candidates and decisions as slice_box (its box contains every kept
 // voxel whatever the last-bit rounding of its start).
@@ -730,8 +731,9 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     const float pm = (float)(p.patch - 1);
     const float nxm = (float)(t.nx - 1), nym = (float)(t.ny - 1);
     const float wx0 = (float)b.x0, wx1 = (float)b.x1, wy0 = (float)b.y0, wy1 = (float)b.y1;
-    const float sgn = POS ? 1.0f : (scale < 0.0f ? -1.0f : 1.0f);
-    const float cthr = ev.thr * ev.cw + __log2f(fabsf(tof ? p.tofk * scale : scale));
+    const float ts = tof ? p.tofk * scale : scale;
+    const float mul = POS ? 1.0f : ts;
+    const float cthr = POS ? ev.thr * ev.cw + __log2f(fabsf(ts)) : ev.thr * ev.cw;
     // LDS byte offset of voxel (X, Y) of slice s (y fastest): lsl(s) + 8 (X Wy + Y)
     const int wy8 = 8 * g.Wy;
     const int sstep = 8 * g.Wx * g.Wy;
@@ -794,7 +796,7 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
                 const int k = __builtin_ctz(m);
                 const int i = k % BX, j = k / BX;
                 if (inside_exact(p, ev, s, c.ix0 + ib + i, c.iy0 + jb + j)) {
-                    const float w = sgn * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
+                    const float w = mul * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
                     atomicAdd(reinterpret_cast<double *>(base + a0 + i * wy8 + 8 * j), (double)w);
                 }
             }
@@ -802,7 +804,7 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
 #pragma unroll
         for (int k = 0; k < NC; k++) {
             if (dt[k] < -kThrMargin) {
-                const float w = sgn * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
+                const float w = mul * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
                 atomicAdd(reinterpret_cast<double *>(base + a0 + (k % BX) * wy8 + 8 * (k / BX)),
                           (double)w);
             }
@@ -1003,7 +1005,8 @@ __device__ __forceinline__ void flush_tile(const TorParams &p, const TileGeom &g
 // stored in the event records (the OSEM step of a plan), not p.val.
 // ONE: every listing's event walks the NB x (NB - 1) box (a plan whose
 // events all have box shape 1); the other walks are left out of the kernel.
-template <int MODE, int NB, bool VREC = false, bool ONE = false>
+// FOLD: the scale in the weights' exponent (scatter_box_yf).
+template <int MODE, int NB, bool VREC = false, bool ONE = false, bool FOLD = MODE == kBack>
 __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom &g,
                                               const TileChunk &ch,
                                               const int *__restrict__ list,
@@ -1054,7 +1057,8 @@ __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom
         }
         if (go) {
             constexpr int NBB = NB > 1 ? NB : 2;
-            constexpr bool POS = MODE == kBack; // scale 1/v with v > 1e-7
+            constexpr bool POS = FOLD; // scale 1/v with v > 1e-7
+            static_assert(!FOLD || MODE == kBack, "only a positive scale has a logarithm");
             const int shape = box_shape<NB>(t);
             static_assert(!ONE || NB > 0, "the single walk is a box walk");
             if (ONE || (NB > 0 && shape == 1))

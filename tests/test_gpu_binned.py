@@ -133,3 +133,28 @@ def test_special_values_and_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert _rel(c, d) <= 1e-5
+
+
+def test_adjoint_of_values_far_from_one():
+    """A power-of-two factor of one event's value scales every weight exactly
+    (the tile sums one event in FP64, each voxel is flushed once)."""
+    grid, size = (40, 40, 36), (80.0, 80.0, 72.0)
+    lors, _ = _events(40_000, size, 13)
+    like = torch.empty(grid[::-1], device=DEV)
+    args = (grid, (0.0, 0.0, 0.0), size, *MODEL, 4.0, False)
+    g = torch.zeros(40_000, device=DEV)
+    g[1234] = -1.25
+    a = ops.backprojection_adjoint(like, lors, g, *args)
+    b = ops.backprojection_adjoint(like, lors, g * 2.0 ** -90, *args)
+    assert bool((a < 0).any()) and torch.equal(a, b * 2.0 ** 90)
+
+
+def test_negative_tof_bin():
+    """The weights' sign follows the TOF bin's, as in the direct scatter."""
+    grid, size = (40, 40, 36), (80.0, 80.0, 72.0)
+    lors, v = _events(40_000, size, 17)
+    like = torch.empty(grid[::-1], device=DEV)
+    args = (grid, (0.0, 0.0, 0.0), size, -6.0, MODEL[1], 4.0, False)
+    b = ops.backprojection(like, lors, v, *args)
+    d = ops.backprojection(like, lors, v, *args, schedule=(1, 256))
+    assert bool((d < 0).any()) and _rel(b, d) <= 1e-5
