@@ -16,12 +16,13 @@ Row order inside a group is the reference's: ascending event index
 
 float32 and float64 rows on a GPU go through the HIP kernels
 (srfx_split_lors_*, srfx_locality_sort), which give the same bits; other rows
-(host tensors, other types, rows that require a gradient) through the torch
-operations below.
+(host tensors, other types, rows that carry a gradient or a tangent, calls under
+stream capture) through the torch operations below.
 """
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -102,7 +103,9 @@ def _as64(lors, ncols):
 
 def _native(t):
     return (type(t) is torch.Tensor and t.device.type == "cuda" and not t.requires_grad
-            and t.dim() == 2 and t.numel() > 0)
+            and t.dim() == 2 and t.numel() > 0 and not t.is_neg()
+            and forward_ad.unpack_dual(t).tangent is None
+            and not torch.cuda.is_current_stream_capturing())
 
 
 SPLIT_ROWS = 1024  # rows per workgroup of srfx_split_lors_count

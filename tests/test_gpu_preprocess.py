@@ -4,6 +4,7 @@ row counts around a workgroup's, both row types and several layouts."""
 import numpy as np
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from srf_amd import preprocess as P
 from tests.test_preprocess import _events
@@ -70,3 +71,16 @@ def test_locality_order(cuda, n, K):
     assert torch.equal(P.locality_order(soa, K, 1.5), want)
     out, orders = P.reorder_groups({"x": soa}, K, {"x": 1.5})
     assert torch.equal(orders["x"], want) and torch.equal(out["x"], soa[:, want])
+
+
+def test_rows_with_a_tangent(cuda):
+    """Forward-mode rows keep their tangent."""
+    rows = torch.from_numpy(_rows(300, 8)).to(cuda)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(rows, torch.ones_like(rows))
+        got = P.recon_process(dual, 530.0)
+        want = P.recon_process(rows, 530.0)
+        for a in "xyz":
+            primal, tangent = forward_ad.unpack_dual(got[a])
+            assert torch.equal(primal, want[a])
+            assert tangent is not None and bool((tangent[0] == 1).any())
