@@ -376,6 +376,19 @@ int srfx_locality_sort(const float *soa, int64_t n, int64_t ld, int32_t ncols,
                        int32_t nb_subsets, double center_z, double zc_bin, double slope_bin,
                        double pos_bin, float *out, int64_t *order, void *stream);
 
+/* srfx_tor_plan_osem_subset of up to three plans (the axis groups of one
+ * subset) together: bp += sum over the plans of A^T (1 / (A image)), one launch
+ * per kernel for all of them.  image and bp are laid out as each plan's grid
+ * says; frames is scratch for the plans' op-frame copies of the image, gx * gy *
+ * gz floats each.  flags: SRFX_ACCUMULATE.  SRFX_EUNSUPPORTED, before any device
+ * work, for plans of different walks (candidate boxes), of another workgroup
+ * size than 256, with frames beyond SRFX_IMAGE_OP_FRAME's fast gathers (2^31
+ * bytes, 2^24 voxels a slice), or of so many events (524288 in all, 65536 with
+ * tubes wider than four voxels) that each fills the chip: run them one by one,
+ * on streams of their own. */
+int srfx_tor_plan_osem_groups(const srfx_tor_plan *plans, int32_t nplans, const float *image,
+                              float *frames, float *bp, uint32_t flags, void *stream);
+
 /* Tiled Siddon backprojection over a fixed LOR set (no counterpart in the
  * reference, whose BackRayTracing adds every segment to the image with its
  * own atomic, siddon.cu.cc:339-381; the ops compute what

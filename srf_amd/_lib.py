@@ -147,6 +147,7 @@ _PROTOS = {
     "srfx_siddon_plan_backproject_adjoint": [_P, _P, _P, _U32, _P],
     "srfx_siddon_plan_osem_subset": [_P, _P, _P, _P, _U32, _P],
     "srfx_siddon_plan_projection": [_P, _P, _P],
+    "srfx_tor_plan_osem_groups": [ctypes.POINTER(_P), _I32, _P, _P, _P, _U32, _P],
     "srfx_split_lors_count": [_P, _I64, _I64, _I64, _I32, _P, _P, _P],
     "srfx_split_lors_fill": [_P, _I64, _I64, _I64, _I32, _I32, _I32, _D, _P, _P,
                              ctypes.POINTER(_P), ctypes.POINTER(_I64), ctypes.POINTER(_P), _P],
@@ -192,6 +193,17 @@ def call(name, *args):
     if status != SRFX_OK:
         raise SrfxError(name, status, lib.srfx_strerror(status).decode())
     return status
+
+
+def try_call(name, *args):
+    """call, but False where the library does not support the arguments."""
+    lib = load()
+    status = getattr(lib, name)(*args)
+    if status == SRFX_EUNSUPPORTED:
+        return False
+    if status != SRFX_OK:
+        raise SrfxError(name, status, lib.srfx_strerror(status).decode())
+    return True
 
 
 def make_grid(shape, center, size, stride=(0, 0, 0)):

@@ -15,6 +15,7 @@ import torch
 from . import _lib
 from .data import Image, ListModeData, ListModeDataSplit
 from .ops import _check_dev, _ptr, _soa, _stream, _vec
+from .plan import TorPlan
 
 # Axis permutation that brings the world image into a group's frame
 # (split_lors.py:54-61); the op frame is the permuted image's axes reversed.
@@ -217,8 +218,8 @@ class SplitLoRsModel:
 
     @staticmethod
     def _check_plan_layout(plan, t):
-        if list(plan.strides) != [int(v) for v in group_frame(
-                t.shape, plan.center, plan.size, t.stride(), plan.axis)[3]]:
+        st = t.stride()
+        if plan.strides != tuple(st[k] for k in PERM[plan.axis][::-1]):
             raise ValueError("image layout differs from the one the plan was built for")
 
     def _source(self, image, a):
@@ -306,10 +307,16 @@ class SplitLoRsModel:
         if out is None:
             out = torch.zeros_like(x)
         if plans is not None:
-            # the groups' steps run concurrently (their scatters add into out
-            # with atomics)
+            # the groups' steps share their launches or run concurrently (their
+            # scatters add into out with atomics)
             steps = [(a, self._planned(plans, a, len(data[a]), out)) for a in self.AXIS
                      if len(data[a])]
+            if (steps and self.stage_frames and self.schedule.get("projection") is None
+                    and x.data_ptr() != out.data_ptr()):
+                for a, pl in steps:
+                    self._check_plan_layout(pl, x)
+                if TorPlan.osem_groups([pl for _, pl in steps], x, out):
+                    return Image(out, image.center, image.size)
             _concurrent([lambda a=a, pl=pl: self.plan_osem_group(pl, x, out, a)
                          for a, pl in steps], (x, out))
             return Image(out, image.center, image.size)

@@ -248,6 +248,28 @@ class TorPlan:
                   _stream())
         return out
 
+    @staticmethod
+    def osem_groups(plans, image, out):
+        """Add the backprojections of 1/p of several plans' events (the axis
+        groups of one subset; image and out laid out as the plans were built
+        for) to out, the plans in one launch per kernel
+        (srfx_tor_plan_osem_groups).  False, with nothing done, for plans that
+        cannot share a launch."""
+        if len(plans) > 3:
+            return False
+        _check_dev(image, "image")
+        _check_dev(out, "out")
+        layout = sorted(zip(image.stride(), image.shape))
+        nvox = 0
+        for pl in plans:
+            if sorted(zip(pl.strides, pl.grid)) != layout:
+                raise ValueError(f"image must have a plan's {pl.grid} voxels and its strides")
+            nvox += pl.grid[0] * pl.grid[1] * pl.grid[2]
+        frames = torch.empty(nvox, dtype=torch.float32, device=image.device)
+        hs = (ctypes.c_void_p * len(plans))(*[pl._h.value for pl in plans])
+        return _lib.try_call("srfx_tor_plan_osem_groups", hs, len(plans), _ptr(image),
+                             _ptr(frames), _ptr(out), _lib.SRFX_ACCUMULATE, _stream())
+
     def scales(self):
         """The backprojection scales the last OSEM step stored in the event
         records: 1/p for p > 1e-7, else 0 (float32 [n])."""
