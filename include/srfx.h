@@ -383,9 +383,8 @@ int srfx_locality_sort(const float *soa, int64_t n, int64_t ld, int32_t ncols,
  * gz floats each.  flags: SRFX_ACCUMULATE.  SRFX_EUNSUPPORTED, before any device
  * work, for plans of different walks (candidate boxes), of another workgroup
  * size than 256, with frames beyond SRFX_IMAGE_OP_FRAME's fast gathers (2^31
- * bytes, 2^24 voxels a slice), or of so many events (524288 in all, 65536 with
- * tubes wider than four voxels) that each fills the chip: run them one by one,
- * on streams of their own. */
+ * bytes, 2^24 voxels a slice), or of so many events (524288 in all) that each
+ * fills the chip: run them one by one, on streams of their own. */
 int srfx_tor_plan_osem_groups(const srfx_tor_plan *plans, int32_t nplans, const float *image,
                               float *frames, float *bp, uint32_t flags, void *stream);
 

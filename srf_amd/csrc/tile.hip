@@ -306,10 +306,9 @@ struct PlanSet {
 
 // Order chunks by length, longest first, in steps of an eighth of a full chunk
 // and stably within one (neighbouring tiles share walk records): the last
-// workgroups to run are short ones.  Box walks: an iteration over 8M events at 200 x
-// 200 x 100 6540 -> 6420 us, over 6M at 256 x 256 x 160 7740 -> 7575.  Chord walks
-// keep the order of the windows: 181 x 175 x 83, 1M events, plans and one iteration
-// 7280 us, longest first 7520.
+// workgroups to run are short ones.  An iteration over 8M events at 200 x 200 x 100
+// 6540 -> 6420 us, over 6M at 256 x 256 x 160 7740 -> 7575; a subset of 500k events
+// with an 8 mm tube, 200 x 200 x 100, 1288 -> 1227.
 void longest_first(std::vector<TileChunk>::iterator a, std::vector<TileChunk>::iterator b, int chunk)
 {
     const int step = std::max(1, chunk / 8);
@@ -523,8 +522,7 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
                         ch.push_back(TileChunk{t, o[t] + q,
                                                c[t] - q < ps.chunk ? c[t] - q : ps.chunk, 0});
             l.nch[k] = (int)(ch.size() - before);
-            if (ps.pls[k]->p.box > 0)
-                longest_first(ch.begin() + before, ch.end(), ps.chunk);
+            longest_first(ch.begin() + before, ch.end(), ps.chunk);
         }
     }
     {

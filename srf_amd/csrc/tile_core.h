@@ -812,7 +812,77 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     }
 }
 
-// The scatter of one listing whose box is larger than the compiled one: the
+// The scatter of one listing of a plan whose events' boxes fit no compiled one
+// (NB = 0): the row walk, as slice_rows_frame (figures there).  Exponents and
+// decisions as scatter_box_yf's.
+__device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGeom &g,
+                                                const TileBox &b, const Event &ev, const Track &t,
+                                                bool tof, float scale, int s0, int s1, double *lds)
+{
+    const float eps = 1.0e-4f;
+    const float ts = tof ? p.tofk * scale : scale;
+    const float c0 = ev.thr * ev.cw;
+    const int wy8 = 8 * g.Wy;
+    const int sstep = 8 * g.Wx * g.Wy;
+    int lsl = (s0 - b.sa) * sstep - 8 * (b.x0 * g.Wy + b.y0);
+    char *const base = reinterpret_cast<char *>(lds);
+    for (int s = s0; s <= s1; s++, lsl += sstep) {
+        Cross c;
+        cross_at(p, ev, t, s, c);
+        const double sd = (double)s;
+        const float cexp = tof ? c0 + (float)fma(fma(t.tc2, sd, t.tc1), sd, t.tc0) : c0;
+        // clipped to the patch and the window (which lies inside the image)
+        const int ib0 = (int)ceilf((c.dx0 - t.hx) * p.rfinter_x - eps);
+        const int jb0 = (int)ceilf((c.dy0 - t.dymax) * p.rfinter_y - eps);
+        const int jb = max(max(0, jb0), b.y0 - c.iy0);
+        const int ie = min(min(p.patch - 1, ib0 + t.nx - 1), b.x1 - c.ix0);
+        const int je = min(min(p.patch - 1, jb0 + t.ny - 1), b.y1 - c.iy0);
+        for (int ib = max(max(0, ib0), b.x0 - c.ix0); ib <= ie; ib += kRowCols) {
+            float cx2[kRowCols], cux[kRowCols];
+#pragma unroll
+            for (int k = 0; k < kRowCols; k++) {
+                col_terms(voxel_offset(c.dx0, ib + k, p.finter_x), ev.ux, cx2[k], cux[k]);
+                cx2[k] = ib + k <= ie ? cx2[k] : INFINITY; // neither kept nor near
+            }
+            int a = lsl + __mul24(c.ix0 + ib, wy8) + 8 * (c.iy0 + jb);
+            for (int j = jb; j <= je; j++, a += 8) {
+                float dyt, uydy, dt[kRowCols], gap = INFINITY;
+                row_terms(voxel_offset(c.dy0, j, p.finter_y), ev.uy, ev.thr, dyt, uydy);
+#pragma unroll
+                for (int k = 0; k < kRowCols; k++) {
+                    dt[k] = tube_dt(cx2[k], cux[k], dyt, uydy);
+                    gap = fminf(gap, fabsf(dt[k]));
+                }
+                if (gap <= kThrMargin) {
+                    // rare: the reference's FP64 decision, one voxel at a time; a
+                    // kept one is added here
+                    uint32_t near = 0;
+#pragma unroll
+                    for (int k = 0; k < kRowCols; k++)
+                        near |= (uint32_t)(fabsf(dt[k]) <= kThrMargin) << k;
+                    for (uint32_t m = (uint32_t)opaque((int)near); m; m &= m - 1) {
+                        const int k = __builtin_ctz(m);
+                        if (inside_exact(p, ev, s, c.ix0 + ib + k, c.iy0 + j)) {
+                            const float d = voxel_dt(ev, voxel_offset(c.dx0, ib + k, p.finter_x),
+                                                     voxel_offset(c.dy0, j, p.finter_y));
+                            const float w = ts * __builtin_amdgcn_exp2f(fmaf(d, ev.cw, cexp));
+                            atomicAdd(reinterpret_cast<double *>(base + a + k * wy8), (double)w);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < kRowCols; k++) {
+                    if (dt[k] < -kThrMargin) {
+                        const float w = ts * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
+                        atomicAdd(reinterpret_cast<double *>(base + a + k * wy8), (double)w);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The scatter of one listing whose box is larger than its plan's compiled one: the
 // clipped chord walk of each slice into the y-fastest tile.  The scale rides
 // in amp (one product per slice, not per voxel), with the TOF constant folded
 // into it once.
@@ -1065,6 +1135,8 @@ __device__ __forceinline__ void scatter_chunk(const TorParams &p, const TileGeom
                 scatter_box_yf<NBB, NBB - 1, POS>(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
             else if (NB > 0 && shape == 2)
                 scatter_box_yf<NBB, NBB, POS>(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
+            else if (NB == 0)
+                scatter_rows_yf(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
             else
                 scatter_chords(p, g, b, ev, t, tof, scale, s0, s1, ldsd);
         }
