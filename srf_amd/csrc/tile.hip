@@ -311,10 +311,20 @@ struct PlanSet {
 // with an 8 mm tube, 200 x 200 x 100, 1288 -> 1227.
 void longest_first(std::vector<TileChunk>::iterator a, std::vector<TileChunk>::iterator b, int chunk)
 {
+    // a counting sort: a stable_sort of the 11,000 chunks of eight plans took 0.25 ms
     const int step = std::max(1, chunk / 8);
-    std::stable_sort(a, b, [step](const TileChunk &x, const TileChunk &y) {
-        return x.count / step > y.count / step;
-    });
+    const std::vector<TileChunk> in(a, b);
+    size_t at[16] = {}; // chunk / step < 16
+    for (const TileChunk &c : in)
+        at[c.count / step]++;
+    size_t before = 0;
+    for (int k = 15; k >= 0; k--) {
+        const size_t n = at[k];
+        at[k] = before;
+        before += n;
+    }
+    for (const TileChunk &c : in)
+        a[at[c.count / step]++] = c;
 }
 
 // Build every set of `sets` in shared phases: the count passes of all sets,

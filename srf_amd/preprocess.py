@@ -244,6 +244,8 @@ def locality_order(soa, nb_subsets, center_z=0.0):
     if _sortable(soa, nb_subsets):
         return _locality_sort(soa, nb_subsets, center_z, False)[1]
     n = soa.shape[1]
+    if n == 0 and soa.shape[0] >= 9:
+        return torch.empty(0, dtype=torch.int64, device=soa.device)
     key = locality_key(soa, center_z)
     order = torch.empty(n, dtype=torch.int64, device=soa.device)
     for k in range(nb_subsets):
