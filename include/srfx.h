@@ -59,8 +59,8 @@ enum srfx_status {
 /* TOR ops: launch schedule.  Lanes that share one event (its crossed slices
  * interleaved between them): SRFX_LPE_1, SRFX_LPE_4, SRFX_LPE_16; without a
  * flag 16 for up to 24576 events, 4 for up to 131072 and one beyond, except
- * the projection of a plan's OSEM step (srfx_tor_plan_osem_subset), which
- * takes four beyond 24576.
+ * projections with tubes wider than four voxels and the projection of a plan's
+ * OSEM step (srfx_tor_plan_osem_subset), which take four beyond 24576.
  * Threads per block: SRFX_BLOCK_256 (default), SRFX_BLOCK_64, SRFX_BLOCK_128.
  * Results agree to FP32 rounding across schedules.
  * Without any schedule flag a large scatter (backprojection, adjoint, Maplors,
@@ -69,8 +69,8 @@ enum srfx_status {
  * workspace of up to 256 MiB from the device's memory pool (a stream under
  * capture, or a failed allocation, keeps the kernels without workspace).
  * Likewise the projection of more than 131072 events over an image of 10 MB
- * and up (4 MB with tubes wider than four voxels) walks the events in a
- * locality order formed on the device (up to 156 MiB of workspace). */
+ * and up walks the events in a locality order formed on the device (up to 156
+ * MiB of workspace). */
 #define SRFX_LPE_SHIFT 4
 #define SRFX_LPE_1 (1u << SRFX_LPE_SHIFT)
 #define SRFX_LPE_4 (2u << SRFX_LPE_SHIFT)

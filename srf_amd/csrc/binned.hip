@@ -412,17 +412,17 @@ int launch_sorted(const TorParams &p, float4 *rec, hipStream_t st)
 
 // Where ordering the events first pays: from 131073 events on (below, lanes
 // that share an event hide the gathers' latency and the four ordering kernels
-// are launch-bound) over images that the gathers of a box walk miss L2 on, or
-// with chord walks, whose patches take more lines.  Events in time order, one
+// are launch-bound) over images whose gathers miss L2.  Events in time order, one
 // lane per event against this path, us: 200 x 200 x 100 x 200k events 298 / 190,
 // x 1M 1165 / 607; 256 x 256 x 160 x 1M 1989 / 798; 181 x 175 x 83 x 400k 380 / 271;
-// 160 x 160 x 80 (8.2 MB) x 400k 213 / 250; chords: 128 x 128 x 64 x 400k 1171 /
-// 650, 181 x 175 x 83 x 1M 4449 / 2112.  Events that come in locality order
-// already, same columns: 197 / 187, 565 / 642, 1112 / 838, 241 / 290, 180 / 258,
-// 763 / 661, 3145 / 2155.
+// 160 x 160 x 80 (8.2 MB) x 400k 213 / 250.  Events that come in locality order
+// already, same columns: 197 / 187, 565 / 642, 1112 / 838, 241 / 290, 180 / 258.
+// Tubes wider than four voxels, four lanes per event against this path: 181 x 175
+// x 83 x 280k 672 / 511, x 600k 1301 / 847; 150 x 150 x 64 (5.8 MB) x 280k 326 /
+// 379, x 600k 607 / 619; 128 x 128 x 64 x 600k 523 / 568.
 constexpr int64_t kSortedEvents = 131073;
-constexpr int64_t kSortedBox = 10000000, kSortedChord = 4000000; // bytes of the image
-constexpr int64_t kSortedPiece = (int64_t)1 << 20;               // 151 MB of records
+constexpr int64_t kSortedBytes = 10000000; // of the image
+constexpr int64_t kSortedPiece = (int64_t)1 << 20; // 151 MB of records
 
 } // namespace
 
@@ -433,7 +433,7 @@ int sorted_project(const TorParams &p, uint32_t flags, hipStream_t st, bool *don
                                (3u << SRFX_SLAB_SHIFT) | SRFX_FULL_PATCH;
     const int64_t bytes = (int64_t)4 * p.gx * p.gy * p.gz;
     if ((flags & sched) || p.n < kSortedEvents ||
-        bytes < (p.box ? kSortedBox : kSortedChord) || !workspace_ok(st))
+        bytes < kSortedBytes || !workspace_ok(st))
         return SRFX_OK;
     const int64_t piece = std::min<int64_t>(p.n, kSortedPiece);
     const size_t rb = align256(sizeof(float4) * kWalkF4 * (size_t)piece);

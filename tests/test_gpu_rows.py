@@ -1,6 +1,6 @@
 """The row walk of wide tubes (boxes of more than four voxels): one and several
 blocks of columns, images narrower than a block, patches over every image edge,
-against the FP64 oracle and the untiled chord walk."""
+against the FP64 oracle, the untiled scatter and the whole patch."""
 import numpy as np
 import pytest
 import torch
@@ -50,8 +50,11 @@ def test_row_walk(grid, pitch, kw, slope, model):
     plan = TorPlan(L, *args, kw, False, *model)
     assert plan.walks()[0] == 0
     p = plan.projection(X, op_frame=True)
-    untiled = ops.projection(L, X, *args, kw, False, *model)
+    untiled = ops.projection(L, X, *args, kw, False, *model, full_patch=True)
     assert _rel(p, untiled) <= 1e-5
+    for schedule in (None, (1, 256), (4, 64)):
+        assert _rel(ops.projection(L, X, *args, kw, False, *model, schedule=schedule),
+                    untiled) <= 1e-5
     ref = torch.from_numpy(O.tor_project(lors, x, *args, kw, False, *model, prec="f64"))
     if model[1] > 1.0:
         assert _rel(p.cpu(), ref.reshape(-1)) <= 1e-5

@@ -41,7 +41,7 @@ def _check(a, b):
     ((190, 120, 112), 2.0, 4.0, 131_073, TOF),      # 3 x 3 box, first sorted size
     ((190, 120, 112), 2.0, 4.0, 140_001, NO_TOF),
     ((190, 120, 112), 1.5, 4.0, 131_137, TOF),      # 4 x 4 box
-    ((128, 100, 80), 2.0, 12.0, 131_073, TOF),      # chord walks
+    ((160, 140, 120), 2.0, 12.0, 131_073, TOF),     # row walks
     ((190, 120, 112), 4.0, 4.0, (1 << 20) + 77, TOF),  # two pieces
 ])
 def test_sorted_projection_matches(grid, pitch, kw, n, model):
