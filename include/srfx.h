@@ -382,9 +382,8 @@ int srfx_locality_sort(const float *soa, int64_t n, int64_t ld, int32_t ncols,
  * says; frames is scratch for the plans' op-frame copies of the image, gx * gy *
  * gz floats each.  flags: SRFX_ACCUMULATE.  SRFX_EUNSUPPORTED, before any device
  * work, for plans of different walks (candidate boxes), of another workgroup
- * size than 256, with frames beyond SRFX_IMAGE_OP_FRAME's fast gathers (2^31
- * bytes, 2^24 voxels a slice), or of so many events (524288 in all) that each
- * fills the chip: run them one by one, on streams of their own. */
+ * size than 256, or with frames beyond SRFX_IMAGE_OP_FRAME's fast gathers (2^31
+ * bytes, 2^24 voxels a slice): run them one by one. */
 int srfx_tor_plan_osem_groups(const srfx_tor_plan *plans, int32_t nplans, const float *image,
                               float *frames, float *bp, uint32_t flags, void *stream);
 

@@ -13,16 +13,6 @@ namespace {
 
 constexpr int kMaxGroups = 3;
 
-// Events of all groups up to which they share launches.  A small subset's step is
-// bound by its launches: three per group, forked to a stream each and joined,
-// took the host 118 us, here one call and three launches in all.  us per subset,
-// groups on streams of their own against together: 96 x 96 x 48, 3000 events
-// 155 / 53, 50k 132 / 79, 400k 190 / 173; 200 x 200 x 100, 3000 130 / 74, 100k
-// 188 / 184, 400k 393 / 388, 1M 786 / 796; 8 mm tube, 181 x 175 x 83, 250k 669 /
-// 650, 200 x 200 x 100, 500k 1227 / 1174.  Beyond, one group's projection beside
-// the other's scatter fills the chip better.
-constexpr int64_t kTogether = 524288;
-
 // One group's plan: its parameters (img: the op frame, out: the
 // backprojection), and where its workgroups start in the launches.
 struct GroupJob {
@@ -137,17 +127,14 @@ extern "C" int srfx_tor_plan_osem_groups(const srfx_tor_plan *plans, int32_t npl
     GroupSet s{};
     s.n = n;
     unsigned sh = 0;
-    int64_t events = 0, most = 0;
+    int64_t most = 0;
     int one = 1;
     for (int k = 0; k < n; k++) {
         sh = std::max(sh, (unsigned)(sizeof(double) * pl[k]->g.S * pl[k]->g.Wx * pl[k]->g.Wy));
-        events += pl[k]->p.n;
         most = std::max(most, pl[k]->p.n);
         one &= pl[k]->one;
     }
     const int box = pl[0]->p.box;
-    if (events > kTogether)
-        return SRFX_EUNSUPPORTED;
     one = (box == 3 && one && 5u * sh <= kCuLds) || (box == 4 && one && 4u * sh <= kCuLds);
     const bool small = lanes_per_event(most) == 16;
     const int lpe = small ? 16 : 4;

@@ -521,7 +521,6 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
                         ch.push_back(TileChunk{t, o[t] + q,
                                                c[t] - q < ps.chunk ? c[t] - q : ps.chunk, 0});
             l.nch[k] = (int)(ch.size() - before);
-            longest_first(ch.begin() + before, ch.end(), ps.chunk);
         }
     }
     {
@@ -548,7 +547,6 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
                 srfx_tor_plan_s *pl = ps.pls[k];
                 pl->chunks = (TileChunk *)blk1 + c0;
                 pl->nchunks = l.nch[k];
-                pl->hchunks.assign(ch.begin() + c0, ch.begin() + c0 + l.nch[k]);
                 c0 += l.nch[k];
                 pl->list = (int *)(blk1 + list_off[j]);
                 pl->nlist = l.totals[k];
@@ -565,8 +563,16 @@ int plan_build_sets(const std::vector<PlanSet> &sets, hipStream_t st)
     }
     if ((rc = launch(true)))
         goto done;
-    // the chunk table, read by the sort only: its copy from pageable memory
-    // is staged while the fill pass runs
+    // the chunk table, read by the sort only: put in order and its copy from
+    // pageable memory staged while the fill pass runs
+    for (int q = 0; q < S; q++) {
+        auto c = ch.begin() + L[q].ch0;
+        for (int k = 0; k < sets[q].K; k++) {
+            longest_first(c, c + L[q].nch[k], sets[q].chunk);
+            sets[q].pls[k]->hchunks.assign(c, c + L[q].nch[k]);
+            c += L[q].nch[k];
+        }
+    }
     if (!ch.empty() && hipMemcpyAsync(blk1, ch.data(), sizeof(TileChunk) * ch.size(),
                                       hipMemcpyHostToDevice, st) != hipSuccess) {
         rc = SRFX_ELAUNCH;

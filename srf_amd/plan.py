@@ -25,7 +25,7 @@ from . import _lib
 from .ops import _check_dev, _geom, _ptr, _soa, _stream, _vec
 
 DEFAULT_TILE = (12, 32, 10)
-# Chord walks (events whose candidate box would be wider than 4 voxels) list
+# Row walks (events whose candidate box would be wider than 4 voxels) list
 # fewer (event, tile) pairs in deeper windows, and have no single-walk kernel
 # to fit five workgroups per CU.
 CHORD_TILE = (12, 32, 12)
@@ -34,9 +34,21 @@ CHORD_TILE = (12, 32, 12)
 def default_tile(grid, size, kernel_width):
     """The default tile of a plan over a frame of ``grid`` voxels spanning
     ``size`` mm at ``kernel_width``: DEFAULT_TILE for the candidate-box
-    walks, CHORD_TILE for the chord walk."""
+    walks, CHORD_TILE for the row walk of wider tubes."""
     return DEFAULT_TILE if _lib.tor_patch_info(grid, size, kernel_width)[1] else CHORD_TILE
+
+
 DEFAULT_CHUNK = 2048
+
+# Events of all groups up to which a subset's groups share launches.  A small
+# subset's step is bound by its launches: three per group, forked to a stream each
+# and joined, took the host 118 us, here one call and three launches in all.  us per
+# subset, groups on streams of their own against together: 96 x 96 x 48, 3000 events
+# 155 / 53, 50k 132 / 79, 400k 190 / 173; 200 x 200 x 100, 3000 130 / 74, 100k
+# 188 / 184, 400k 393 / 388, 1M 786 / 796; 8 mm tube, 181 x 175 x 83, 250k 669 /
+# 650, 200 x 200 x 100, 500k 1227 / 1174.  Beyond, one group's projection beside the
+# other's scatter fills the chip better.
+GROUP_EVENTS = 524288
 
 
 class TorPlan:
@@ -254,8 +266,8 @@ class TorPlan:
         groups of one subset; image and out laid out as the plans were built
         for) to out, the plans in one launch per kernel
         (srfx_tor_plan_osem_groups).  False, with nothing done, for plans that
-        cannot share a launch."""
-        if len(plans) > 3:
+        cannot share a launch or have more than GROUP_EVENTS events."""
+        if len(plans) > 3 or sum(pl.n for pl in plans) > GROUP_EVENTS:
             return False
         _check_dev(image, "image")
         _check_dev(out, "out")
