@@ -320,6 +320,7 @@ def main():
         model.osem_subset = timed_tiled
     elif not args.unfused:
         model.osem_subset = timed_osem
+    osem.iterate(image, 1)  # not timed: this stream's frame buffers are allocated
     timings.clear()
     osem.iterate(image, args.steps)
     torch.cuda.synchronize()
