@@ -43,8 +43,8 @@ struct EvChunk {
 
 // Box classes of the batch's jobs: 0 = candidate box 3 with every event on
 // the 3 x 2 box (the single-walk scatter), 1 = other box-3 jobs, 2 = box 4, 3 =
-// chord walk.  Each class has its own work lists and kernels, so that a kernel holds only its class's walk (and
-// its registers).
+// wider tubes (the row walk).  Each class has its own work lists and kernels, so
+// that a kernel holds only its class's walk (and its registers).
 constexpr int kBoxClasses = 4;
 
 inline int box_class(const TorParams &p, bool single_walk)

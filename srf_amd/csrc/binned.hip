@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void bin_direct(TorParams p, const BinState *s
 }
 
 // The tile of a binned pass: that of the plans (30 KB of FP64 LDS, five
-// workgroups per CU; chord walks list fewer pairs in a wider window).
+// workgroups per CU; row walks list fewer pairs in a wider window).
 TileGeom bin_geom(const TorParams &p)
 {
     TileGeom g{};
