@@ -451,13 +451,14 @@ __device__ __forceinline__ double mesh_y(const TorParams &p, int iy)
 // -0.6 +- 4.3 and -0.8 +- 0.7 in 1e-10 of 3.6e-7 and 2.3e-7, projections of 2000
 // -3.4 +- 1.8 of 1.1e-7).  A
 // crossing 2^19 voxels or more away leaves the binade: its floor then reads as
-// 2^19 or more or below -2^19 (a NaN's as the former), outside any grid.
+// 2^19 or more or below -2^19, and the reference's arithmetic decides.
 constexpr double kFixed = 0x1.8p20;
 constexpr unsigned kFixedHi = 0x41380000u; // high word of kFixed
 // Fractions this near an integer (2^-20 voxel, in units of 2^-32) are decided by
 // the reference's own arithmetic: above the error of u for |ax| up to 2^31 voxels,
 // a direction cosine along the slice axis of 1e-7.
 constexpr unsigned kFixedNear = 4096u;
+constexpr unsigned kFixedRange = 1u << 19; // |u| below it stays in the binade
 
 __device__ __forceinline__ void cross_at(const TorParams &p, const Event &ev, const Track &t, int s,
                                          Cross &c)
@@ -474,11 +475,12 @@ __device__ __forceinline__ void cross_at(const TorParams &p, const Event &ev, co
     // far inside kThrMargin
     c.dx0 = fmaf((float)lu, p.fxunit, p.fdx_half);
     c.dy0 = fmaf((float)lw, p.fyunit, p.fdy_half);
-    // Rare: a fraction near an integer, or a crossing left of or below the grid,
-    // where the reference's (int) cast rounds up.  One branch.
+    // Rare: a fraction near an integer, a crossing out of range, or one left of or
+    // below the grid, where the reference's (int) cast rounds up.  One branch.
     const bool near = min(lu + kFixedNear, lw + kFixedNear) < 2u * kFixedNear;
-    if ((int)near | (int)((iu | iw) < 0)) {
-        if (near) {
+    if ((int)near | (int)((unsigned)(iu | iw) >= kFixedRange)) {
+        if (near || max((unsigned)iu + kFixedRange, (unsigned)iw + kFixedRange) >=
+                        2u * kFixedRange) {
             double cx, cy;
             cross_point_exact(p, exact_geom(p, ev), s, cx, cy);
             c.ix0 = (int)__ddiv_rn(__dsub_rn(cx, p.l_bound), p.inter_x) - p.half;

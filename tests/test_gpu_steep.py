@@ -58,3 +58,39 @@ def test_crossing_on_a_voxel_face(kw, axis):
     L, X = torch.from_numpy(lors).to(DEV), torch.from_numpy(x).to(DEV)
     want = O.tor_project(lors, x, *args, prec="f64").reshape(-1)
     assert _rel(ops.projection(L, X, *args, full_patch=True), want) <= TOL
+
+
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("kw", [4.0, 8.0])
+def test_columns_and_rows_beyond_2_to_19(axis, kw):
+    """An image of 2^19 + 2^17 columns (rows): the fixed-point crossing holds 2^19 and
+    the reference's arithmetic takes the rest."""
+    m = (1 << 19) + (1 << 17)
+    pitch = 2.0
+    grid = (m, 4, 3) if axis == 0 else (4, m, 3)
+    size = tuple(g * pitch for g in grid)
+    r = np.random.default_rng(6)
+    n = 300
+    mid = r.uniform(-0.4, 0.4, (n, 3)) * size
+    # columns around 0, around 2^19 and to the end
+    at = np.concatenate([r.uniform(0, 40, 100), (1 << 19) + r.uniform(-40, 40, 100),
+                         m - r.uniform(0, 90000, 100)])
+    mid[:, axis] = np.round(((at - m / 2) * pitch) * 16) / 16
+    d = r.uniform(-0.7, 0.7, (n, 3))
+    d[:, 2] = 1.0
+    t = 8.0
+    p1, p2 = mid - d * t, mid + d * t
+    lors = np.vstack([p1.T, p2.T, mid.T, np.ones((1, n))]).astype(np.float32)
+    x = r.uniform(0.5, 1.5, grid[::-1]).astype(np.float32)
+    args = (grid, (0.0, 0.0, 0.0), size)
+    L, X = torch.from_numpy(lors).to(DEV), torch.from_numpy(x).to(DEV)
+    want = O.tor_project(lors, x, *args, kw, False, 6.0, 1.0e6, prec="f64").reshape(-1)
+    got = ops.projection(L, X, *args, kw, False, 6.0, 1.0e6).cpu().double().numpy().reshape(-1)
+    assert (want > 0).sum() > 250
+    # offsets from the crossing are differences of coordinates near 6e5 mm, FP64 to
+    # 1e-10 mm: the FP32 weights and sums alone, 1e-5
+    assert _rel(got, want) <= 1e-5
+    v = np.ones(n, np.float32)
+    back = O.tor_backproject(lors, v, *args, kw, False, 6.0, 1.0e6, prec="f64").reshape(-1)
+    b = ops.backprojection(X, L, torch.from_numpy(v).to(DEV), *args, 6.0, 1.0e6, kw, False)
+    assert _rel(b, back) <= 1e-5
