@@ -819,7 +819,6 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
                                                 const TileBox &b, const Event &ev, const Track &t,
                                                 bool tof, float scale, int s0, int s1, double *lds)
 {
-    const float eps = 1.0e-4f;
     const float ts = tof ? p.tofk * scale : scale;
     const float c0 = ev.thr * ev.cw;
     const int wy8 = 8 * g.Wy;
@@ -832,8 +831,8 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
         const double sd = (double)s;
         const float cexp = tof ? c0 + (float)fma(fma(t.tc2, sd, t.tc1), sd, t.tc0) : c0;
         // clipped to the patch and the window (which lies inside the image)
-        const int ib0 = (int)ceilf((c.dx0 - t.hx) * p.rfinter_x - eps);
-        const int jb0 = (int)ceilf((c.dy0 - t.dymax) * p.rfinter_y - eps);
+        const int ib0 = box_start(c.dx0, t.hx, p.rfinter_x);
+        const int jb0 = box_start(c.dy0, t.dymax, p.rfinter_y);
         const int jb = max(max(0, jb0), b.y0 - c.iy0);
         const int ie = min(min(p.patch - 1, ib0 + t.nx - 1), b.x1 - c.ix0);
         const int je = min(min(p.patch - 1, jb0 + t.ny - 1), b.y1 - c.iy0);

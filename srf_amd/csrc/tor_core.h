@@ -263,8 +263,13 @@ struct Track {
     float tm;    // cut-off padded so the candidate set contains every kept voxel
     float dymax; // sqrt(tm / q): half height of the ellipse
     float hx;    // sqrt(tm (A + cxy^2 / q)): half width of the ellipse
-    int nx, ny;  // voxel columns / rows any slice's ellipse can span
+    int nx, ny;  // voxel columns / rows any slice's ellipse can span (<= kMaxSpan)
 };
+
+// Largest span of a track: 15 bits, what a walk record holds.  An event nearly
+// parallel to the slices (direction cosine along the slice axis below ~1e-4)
+// spans more; box_start keeps a span cut to kMaxSpan over the whole patch.
+constexpr int kMaxSpan = 0x7fff;
 
 namespace {
 
@@ -300,8 +305,8 @@ __device__ __forceinline__ void make_track(const TorParams &p, const Event &ev,
     t.hx = sqrtf(t.tm * (t.A + t.cxy * t.cxy / t.q));
     // integers in an open interval of length 2h/pitch, with the index
     // rounding allowance of the box start (1e-4) on both ends
-    t.nx = (int)fminf(floorf(2.0f * t.hx * p.rfinter_x + 2.0e-4f), 1.0e6f) + 1;
-    t.ny = (int)fminf(floorf(2.0f * t.dymax * p.rfinter_y + 2.0e-4f), 1.0e6f) + 1;
+    t.nx = (int)fminf(floorf(2.0f * t.hx * p.rfinter_x + 2.0e-4f), (float)(kMaxSpan - 1)) + 1;
+    t.ny = (int)fminf(floorf(2.0f * t.dymax * p.rfinter_y + 2.0e-4f), (float)(kMaxSpan - 1)) + 1;
 }
 
 // Event and track of row e of the raw LOR rows (MODE kMap: 7 columns, else
@@ -1008,6 +1013,17 @@ __device__ __forceinline__ bool slice_gather_inner(const TorParams &p, const Eve
     return true;
 }
 
+// First patch column (row) of the ellipse of half width h (mm) around a crossing
+// point d0 from the centre of column 0, for walks that take the ellipse's last
+// column as this one plus the track's span.  Not before -kMaxSpan / 2: a span
+// of kMaxSpan or more starts further left, and from there kMaxSpan columns
+// reach over every patch; shorter spans start later.
+__device__ __forceinline__ int box_start(float d0, float h, float rinter)
+{
+    const float eps = 1.0e-4f;
+    return (int)fmaxf(ceilf((d0 - h) * rinter - eps), (float)(-kMaxSpan / 2));
+}
+
 // Columns of the row walk: the walk of tubes whose box fits no compiled one
 // (NB = 0), kRowCols candidates of a row at a time.
 constexpr int kRowCols = 6;
@@ -1029,9 +1045,8 @@ __device__ __forceinline__ float slice_rows_frame(const TorParams &p, const Even
     const int P = p.patch;
     if (c.ix0 <= -P || c.ix0 >= p.gx || c.iy0 <= -P || c.iy0 >= p.gy)
         return 0.0f;
-    const float eps = 1.0e-4f;
-    const int ib0 = (int)ceilf((c.dx0 - t.hx) * p.rfinter_x - eps);
-    const int jb0 = (int)ceilf((c.dy0 - t.dymax) * p.rfinter_y - eps);
+    const int ib0 = box_start(c.dx0, t.hx, p.rfinter_x);
+    const int jb0 = box_start(c.dy0, t.dymax, p.rfinter_y);
     const int ie = min(min(P, p.gx - c.ix0), ib0 + t.nx) - 1;
     const int jb = max(max(0, -c.iy0), jb0);
     const int je = min(min(P, p.gy - c.iy0), jb0 + t.ny) - 1;
