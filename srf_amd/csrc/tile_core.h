@@ -711,11 +711,12 @@ __device__ __forceinline__ float window_walk(const TorParams &p, const TileGeom 
 //     (lo, hi) on its first column / row, so the offsets need no integer
 //     round trip; clipped candidates get an infinite term (neither kept nor
 //     near).
-//   * The slice's TOF factor folded into each kept candidate's exponent,
-//     exp2(cw dt + thr cw + TOF quadratic), with POS (a positive scale: the
-//     ratio backprojection) log2(scale tofk) as well; else scale tofk is a
-//     factor of its own, so that a scale far from 1 costs the exponent no
-//     digits.
+//   * With POS (a positive scale: the ratio backprojection of a plan) the
+//     slice's TOF factor and the scale folded into each kept candidate's exponent,
+//     exp2(cw dt + thr cw + TOF quadratic + log2(scale tofk)); else both are
+//     factors, as in the direct scatter: the sum of the exponents has up to two
+//     digits less than each (weights of a TOF set 9 % further off, root mean
+//     square; 20 % in the row walk).
 //   * LDS byte offsets carried from slice to slice.
 // The same candidates and decisions as slice_box (its box contains every kept
 // voxel whatever the last-bit rounding of its start).
@@ -732,7 +733,6 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     const float nxm = (float)(t.nx - 1), nym = (float)(t.ny - 1);
     const float wx0 = (float)b.x0, wx1 = (float)b.x1, wy0 = (float)b.y0, wy1 = (float)b.y1;
     const float ts = tof ? p.tofk * scale : scale;
-    const float mul = POS ? 1.0f : ts;
     const float cthr = POS ? ev.thr * ev.cw + __log2f(fabsf(ts)) : ev.thr * ev.cw;
     // LDS byte offset of voxel (X, Y) of slice s (y fastest): lsl(s) + 8 (X Wy + Y)
     const int wy8 = 8 * g.Wy;
@@ -741,8 +741,13 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     for (int s = s0; s <= s1; s++, lsl += sstep) {
         Cross c;
         cross_at(p, ev, t, s, c);
-        const double sd = (double)s;
-        const float cexp = tof ? cthr + (float)fma(fma(t.tc2, sd, t.tc1), sd, t.tc0) : cthr;
+        float cexp = cthr, mul = 1.0f;
+        if (POS) {
+            const double sd = (double)s;
+            cexp = tof ? cthr + (float)fma(fma(t.tc2, sd, t.tc1), sd, t.tc0) : cthr;
+        } else {
+            mul = tof ? tof_exp(p, ev, t, s) * ts : ts;
+        }
         const float fx0 = (float)c.ix0, fy0 = (float)c.iy0;
         const float ib0 = ceilf(fmaf(c.dx0, p.rfinter_x, -hxr));
         const float jb0 = ceilf(fmaf(c.dy0, p.rfinter_y, -dyr));
@@ -813,14 +818,14 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
 }
 
 // The scatter of one listing of a plan whose events' boxes fit no compiled one
-// (NB = 0): the row walk, as slice_rows_frame (figures there).  Exponents and
-// decisions as scatter_box_yf's.
+// (NB = 0): the row walk, as slice_rows_frame (figures there).  Weights as the
+// chord walk's, the TOF factor and the scale once per slice; decisions as
+// scatter_box_yf's.
 __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGeom &g,
                                                 const TileBox &b, const Event &ev, const Track &t,
                                                 bool tof, float scale, int s0, int s1, double *lds)
 {
-    const float ts = tof ? p.tofk * scale : scale;
-    const float c0 = ev.thr * ev.cw;
+    const float ts = p.tofk * scale;
     const int wy8 = 8 * g.Wy;
     const int sstep = 8 * g.Wx * g.Wy;
     int lsl = (s0 - b.sa) * sstep - 8 * (b.x0 * g.Wy + b.y0);
@@ -828,8 +833,7 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
     for (int s = s0; s <= s1; s++, lsl += sstep) {
         Cross c;
         cross_at(p, ev, t, s, c);
-        const double sd = (double)s;
-        const float cexp = tof ? c0 + (float)fma(fma(t.tc2, sd, t.tc1), sd, t.tc0) : c0;
+        const float amp = tof ? tof_exp(p, ev, t, s) * ts : scale;
         // clipped to the patch and the window (which lies inside the image)
         const int ib0 = box_start(c.dx0, t.hx, p.rfinter_x);
         const int jb0 = box_start(c.dy0, t.dymax, p.rfinter_y);
@@ -864,7 +868,7 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
                         if (inside_exact(p, ev, s, c.ix0 + ib + k, c.iy0 + j)) {
                             const float d = voxel_dt(ev, voxel_offset(c.dx0, ib + k, p.finter_x),
                                                      voxel_offset(c.dy0, j, p.finter_y));
-                            const float w = ts * __builtin_amdgcn_exp2f(fmaf(d, ev.cw, cexp));
+                            const float w = voxel_weight(ev, amp, d);
                             atomicAdd(reinterpret_cast<double *>(base + a + k * wy8), (double)w);
                         }
                     }
@@ -872,7 +876,7 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
 #pragma unroll
                 for (int k = 0; k < kRowCols; k++) {
                     if (dt[k] < -kThrMargin) {
-                        const float w = ts * __builtin_amdgcn_exp2f(fmaf(dt[k], ev.cw, cexp));
+                        const float w = voxel_weight(ev, amp, dt[k]);
                         atomicAdd(reinterpret_cast<double *>(base + a + k * wy8), (double)w);
                     }
                 }
