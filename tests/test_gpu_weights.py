@@ -66,3 +66,34 @@ def test_weights_as_precise_as_the_direct_scatter(pitch, kw):
         d = _rms(ops.backprojection(like, L[:, :m].contiguous(), V, *args, *TOF, kw, False,
                                     schedule=(1, 256)), back)
         assert _rms(plan.backprojection(V), back) <= 1.05 * d
+
+
+@pytest.mark.parametrize("n", [361, 200_000])
+def test_siddon_tof_weights(n):
+    """Values of TOF segments one by one, direct and binned: distance, variance and
+    quotient in FP64, then FP32.  Roundings of 2^-24 / sqrt(12) of a value, root mean
+    square 1.7e-8 at the bottom of a binade to 3.4e-8 at its top: segment length,
+    Gaussian, reciprocal root, their products, weight, bin and scale, eight in all,
+    9e-8 at most, and the exponent's two (the quotient and its product with log2 e, up
+    to 6.5 of a base-2 exponent: 2^-22 ln 2 / sqrt(3) at most, in the outer third of the
+    values), 5e-8 over all: 1.1e-7, with a tenth to spare for the hardware functions'
+    ulp.  The quotient in FP32 makes it 1.5e-7."""
+    grid, size, ts2 = (120, 120, 100), (240.0, 240.0, 220.0), 400.0
+    geo = (grid, (0.0, 0.0, 0.0), size)
+    r = np.random.default_rng(3)
+    x, y = [np.arange(-size[k] / 2 + 6.0, size[k] / 2 - 6.0, 12.0) for k in (0, 1)]
+    x, y = [v.ravel() for v in np.meshgrid(x, y)]  # rays apart: a voxel holds one value
+    m = x.size
+    x, y = x + r.uniform(-2, 2, m), y + r.uniform(-2, 2, m)
+    dx, dy = r.uniform(-2.5, 2.5, (2, m))
+    z = np.full(m, size[2] / 2 + 5)
+    lors = np.vstack([x - dx, y - dy, -z, x + dx, y + dy, z,
+                      r.uniform(-40, 40, m)]).astype(np.float32)
+    g = r.uniform(0.5, 2.0, m).astype(np.float32)
+    ref = O.siddon_backproject_adjoint(lors, g, *geo, 6.0, ts2, prec="f64")
+    assert m == 361 and (ref != 0).sum() > 20000
+    L = torch.from_numpy(np.ascontiguousarray(np.tile(lors, -(-n // m))[:, :n])).to(DEV)
+    G = torch.zeros(n, device=DEV)
+    G[:m] = torch.from_numpy(g).to(DEV)
+    like = torch.empty(grid[::-1], device=DEV)
+    assert _rms(ops.siddon_backprojection_adjoint(like, L, G, *geo, 6.0, ts2), ref) <= 1.25e-7
