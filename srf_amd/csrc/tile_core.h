@@ -740,7 +740,7 @@ __device__ __forceinline__ void scatter_box_yf(const TorParams &p, const TileGeo
     int lsl = (s0 - b.sa) * sstep - 8 * (b.x0 * g.Wy + b.y0);
     for (int s = s0; s <= s1; s++, lsl += sstep) {
         Cross c;
-        cross_at(p, ev, t, s, c);
+        cross_at(p, ev, t, t.ax, s, c);
         float cexp = cthr, mul = 1.0f;
         if (POS) {
             const double sd = (double)s;
@@ -825,6 +825,7 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
                                                 const TileBox &b, const Event &ev, const Track &t,
                                                 bool tof, float scale, int s0, int s1, double *lds)
 {
+    const double ax = wide_start(t);
     const float ts = p.tofk * scale;
     const int wy8 = 8 * g.Wy;
     const int sstep = 8 * g.Wx * g.Wy;
@@ -832,7 +833,7 @@ __device__ __forceinline__ void scatter_rows_yf(const TorParams &p, const TileGe
     char *const base = reinterpret_cast<char *>(lds);
     for (int s = s0; s <= s1; s++, lsl += sstep) {
         Cross c;
-        cross_at(p, ev, t, s, c);
+        cross_at(p, ev, t, ax, s, c);
         const float amp = tof ? tof_exp(p, ev, t, s) * ts : scale;
         // clipped to the patch and the window (which lies inside the image)
         const int ib0 = box_start(c.dx0, t.hx, p.rfinter_x);
@@ -893,10 +894,11 @@ __device__ __forceinline__ void scatter_chords(const TorParams &p, const TileGeo
                                                const TileBox &b, const Event &ev, const Track &t,
                                                bool tof, float scale, int s0, int s1, double *lds)
 {
+    const double ax = wide_start(t);
     const float ts = p.tofk * scale;
     for (int s = s0; s <= s1; s++) {
         Cross c;
-        cross_at(p, ev, t, s, c);
+        cross_at(p, ev, t, ax, s, c);
         const float amp = tof ? tof_exp(p, ev, t, s) * ts : scale;
         window_walk<1, true>(p, g, b, ev, t, c, amp, s, scale, lds);
     }
@@ -911,11 +913,12 @@ __device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom
 {
     constexpr int NBB = NB > 1 ? NB : 2;
     const int shape = box_shape<NB>(t);
+    const double ax = NB > 0 && shape ? t.ax : wide_start(t);
     const int P = p.patch;
     float acc = 0.0f;
     for (int s = s0; s <= s1; s++) {
         Cross c;
-        cross_at(p, ev, t, s, c);
+        cross_at(p, ev, t, ax, s, c);
         const float amp = tof ? tof_factor(p, ev, t, s) : 1.0f;
         if (NB > 0 && shape) {
             PatchIdx idx;

@@ -448,28 +448,38 @@ __device__ __forceinline__ double mesh_y(const TorParams &p, int iy)
 // conversion (seven FP64 conversions and differences a slice before, of ~150
 // instructions; the walks are bound by instruction issue.  OSEM iterations: 8M
 // events at 200 x 200 x 100 6345 -> 6320 us, 6M at 256 x 256 x 160 7470 -> 7344, the
-// batch of 12 at 128 x 128 x 64 1818 -> 1726).  u carries the rounding of ax + 1.5 2^20 and of
-// the step, 2^-32 voxel together, which dx0 and dy0 in FP32 do not resolve, and
-// what ax itself carries: for events nearly parallel to the slices, whose ax is
-// large, 2^-53 of it.  Errors of the walks against 64 bits are those of u in FP64
-// (20 seeds each, difference over its own spread: OSEM over 30k and 200k events
+// batch of 12 at 128 x 128 x 64 1818 -> 1726).  u carries the rounding of
+// ax + 1.5 2^20 and of the step, 2^-32 voxel together, which dx0 and dy0 in FP32
+// do not resolve: the walks' errors against 64 bits are those of u in FP64 (20
+// seeds each, difference over its own spread: OSEM over 30k and 200k events
 // -0.6 +- 4.3 and -0.8 +- 0.7 in 1e-10 of 3.6e-7 and 2.3e-7, projections of 2000
-// -3.4 +- 1.8 of 1.1e-7).  A
-// crossing 2^19 voxels or more away leaves the binade: its floor then reads as
-// 2^19 or more or below -2^19, and the reference's arithmetic decides.
+// -3.4 +- 1.8 of 1.1e-7).  A crossing 2^19 voxels or more away leaves the binade:
+// its floor then reads as 2^19 or more or below -2^19, and the reference's
+// arithmetic decides.
 constexpr double kFixed = 0x1.8p20;
 constexpr unsigned kFixedHi = 0x41380000u; // high word of kFixed
-// Fractions this near an integer (2^-20 voxel, in units of 2^-32) are decided by
-// the reference's own arithmetic: above the error of u for |ax| up to 2^31 voxels,
-// a direction cosine along the slice axis of 1e-7.
-constexpr unsigned kFixedNear = 4096u;
 constexpr unsigned kFixedRange = 1u << 19; // |u| below it stays in the binade
+// Fractions this near an integer (3.7e-9 voxel, in units of 2^-32) are decided by
+// the reference's own arithmetic.  No more: the direct planes of a scanner whose
+// ring pitch is a multiple of the voxel's lie on voxel faces up to the rounding of
+// their FP32 rows (a margin of 1e-6: 6M events at 256 x 256 x 160 7360 -> 8140 us).
+constexpr unsigned kFixedNear = 16u;
+// |ax| and |ay| up to which that margin is above the error of u, ~2^-50 |ax|.
+constexpr double kFixedStart = 0x1p20;
 
-__device__ __forceinline__ void cross_at(const TorParams &p, const Event &ev, const Track &t, int s,
-                                         Cross &c)
+// The start of u of an event that may be nearly parallel to the slices (one whose
+// box fits no compiled one): out of range where the track starts further away.
+__device__ __forceinline__ double wide_start(const Track &t)
+{
+    return fmax(fabs(t.ax), fabs(t.ay)) < kFixedStart ? t.ax : 0x1p1000;
+}
+
+// ax: t.ax, or wide_start(t).
+__device__ __forceinline__ void cross_at(const TorParams &p, const Event &ev, const Track &t,
+                                         double ax, int s, Cross &c)
 {
     const double sd = (double)s;
-    const double u = fma(sd, t.bx, t.ax + kFixed), w = fma(sd, t.by, t.ay + kFixed);
+    const double u = fma(sd, t.bx, ax + kFixed), w = fma(sd, t.by, t.ay + kFixed);
     const int iu = (int)((unsigned)__double2hiint(u) - kFixedHi);
     const int iw = (int)((unsigned)__double2hiint(w) - kFixedHi);
     const unsigned lu = (unsigned)__double2loint(u), lw = (unsigned)__double2loint(w);
@@ -1176,13 +1186,14 @@ __device__ __forceinline__ float walk_event(const TorParams &p, const Event &ev,
 {
     constexpr int NBB = NB > 1 ? NB : 2;
     const int shape = p.full_patch ? 0 : box_shape<NB>(t);
+    const double ax = NB > 0 && shape ? t.ax : wide_start(t);
     const float ts = p.tofk * scale;
     float acc = 0.0f;
     for (int s = s_first; s <= s_last; s += rstep) {
         if (s < s_min)
             continue; // a slice before the event's first (aligned walks)
         Cross c;
-        cross_at(p, ev, t, s, c);
+        cross_at(p, ev, t, ax, s, c);
         // scatters: the scale rides in amp (one product per slice, not per
         // voxel), with the TOF constant folded into it once; gathers: the TOF
         // constant multiplies the walk's sum once, after the loop
