@@ -102,10 +102,10 @@ class SplitLoRsModel:
         return _lib.schedule_flags(self.schedule.get(op))
 
     def autotune(self, image, data, sample=262144, reps=3, ops_=("osem_subset",)):
-        """Time every (lanes_per_event, block) schedule of each op in ``ops_``
-        on the first ``sample`` events of every group of ``data`` and keep the
-        fastest.  Returns {op: {schedule: ms}}."""
-        from .autotune import SCHEDULES, _time
+        """Time the library's own choice (None) and every (lanes_per_event, block)
+        schedule of each op in ``ops_`` on the first ``sample`` events of every
+        group of ``data`` and keep the fastest.  Returns {op: {schedule: ms}}."""
+        from .autotune import CANDIDATES, _time, fastest
         sub = ListModeDataSplit(*[data[a].replace_values(
             None if data[a].values is None else data[a].values[:sample]) for a in self.AXIS])
         for a in self.AXIS:
@@ -115,7 +115,7 @@ class SplitLoRsModel:
             times = {}
             if op == "backprojection":
                 proj = self.projection(image, sub)
-            for sch in SCHEDULES:
+            for sch in CANDIDATES:
                 self.schedule[op] = sch
                 if op == "osem_subset":
                     fn = lambda: self.osem_subset(image, sub)
@@ -124,7 +124,7 @@ class SplitLoRsModel:
                 else:
                     fn = lambda: self.backprojection(proj, image)
                 times[sch] = _time(fn, reps)
-            self.schedule[op] = min(times, key=times.get)
+            self.schedule[op] = fastest(times)
             report[op] = times
         return report
 
