@@ -173,7 +173,7 @@ __global__ __launch_bounds__(64, NB == 3 && LPE <= 4 && T <= 128 ? 5 : 4) void b
         const int i = (q % kParts) * T + r + lane % kRound;
         const bool valid = i < ch.count;
         const int64_t e = (int64_t)ch.start + i;
-        record_project<NB, LPE, true>(job.p, rec, e, sub, valid);
+        record_project<NB, LPE, true, false, true>(job.p, rec, e, sub, valid);
     }
 }
 

@@ -953,7 +953,9 @@ __device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom
 // The lanes of an event are 64 / LPE apart: neighbouring lanes are neighbouring
 // events on the same slice, whose loads share lines (side by side on different
 // slices they never do; 8M events, one iteration, 6430 -> 6345 us).
-template <int NB, int LPE, bool FRAME = false, bool SORTED = false>
+// ALIGN: for events whose order differs from call to call or from plan to plan
+// (locality.hip's places), the same sum whichever events share the wave.
+template <int NB, int LPE, bool FRAME = false, bool SORTED = false, bool ALIGN = SORTED>
 __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, int64_t e,
                                                int sub, bool valid, float *pout = nullptr)
 {
@@ -976,9 +978,7 @@ __device__ __forceinline__ void record_project(const TorParams &p, float4 *rec, 
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1)
         base = min(base, __shfl_xor(base, m, 64));
-    // in an order that differs from call to call, lane sub takes the slices
-    // congruent to it: the same sum whichever events share the wave
-    if (SORTED)
+    if (ALIGN) // lane sub takes the slices congruent to it
         base &= ~(LPE - 1);
     if (any)
         part = walk_event<0, NB, FRAME>(p, ev, t, p.use_tof, 0.0f, base + sub, ev.s_hi, LPE,
