@@ -64,8 +64,9 @@ enum srfx_status {
  * Threads per block: SRFX_BLOCK_256 (default), SRFX_BLOCK_64, SRFX_BLOCK_128.
  * Results agree to FP32 rounding across schedules.
  * Without any schedule flag a large scatter (backprojection, adjoint, Maplors,
- * OSEM pass; ~2.4e6 weights and up) runs binned: its events are listed by image
- * tile on the device and every tile accumulated in LDS, with a stream-ordered
+ * OSEM pass; ~2.4e6 weights and up, ten an event and up; srfx_tor_scatter_rule)
+ * runs binned: its events are listed by image tile on the device and every tile
+ * accumulated in LDS, with a stream-ordered
  * workspace of up to 256 MiB from the device's memory pool (a stream under
  * capture, or a failed allocation, keeps the kernels without workspace).
  * Likewise the projection of more than 131072 events over an image of 10 MB
@@ -198,6 +199,12 @@ int srfx_tor_osem_subset_noalloc(const float *lors, int64_t n, int64_t ld, const
  * output pointer may be NULL.  SRFX_EUNSUPPORTED for P > 16, as the ops. */
 int srfx_tor_patch_info(srfx_grid grid, float kernel_width, int32_t *patch, int32_t *box);
 
+/* Whether a scatter of n events (srfx_tor_backproject, _adjoint, _maplors (model
+ * without TOF), _osem_subset) over a grid runs binned, by the size rule beside
+ * SRFX_LPE_SHIFT: *binned 1 or 0.  Host only: no device work. */
+int srfx_tor_scatter_rule(int64_t n, srfx_grid grid, srfx_tor_model model, uint32_t flags,
+                          int32_t *binned);
+
 /* ------------------------------------------------------------- Siddon --- */
 
 /* Replaces op "Projection" of siddon.so: siddon.cc:14-26, 88-136;
@@ -233,6 +240,10 @@ int srfx_siddon_osem_subset(const float *lors, int64_t n, int64_t ld, const floa
 int srfx_siddon_count_nnz(const float *lors, int64_t n, int64_t ld, srfx_grid grid,
                           float tof_bin, float tof_sigma2, int32_t *nnz_per_event,
                           uint64_t *nnz_total, void *stream);
+
+/* srfx_tor_scatter_rule of the Siddon scatters (~2e6 weights and up). */
+int srfx_siddon_scatter_rule(int64_t n, srfx_grid grid, float tof_bin, float tof_sigma2,
+                             int32_t *binned);
 
 /* ------------------------------------------------------------- Tiled --- */
 

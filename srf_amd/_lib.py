@@ -112,12 +112,14 @@ _PROTOS = {
     "srfx_tor_osem_subset_noalloc": [_P, _I64, _I64, _P, SrfxGrid, SrfxGrid, SrfxTorModel, _P,
                                      _U32, _P],
     "srfx_tor_patch_info": [SrfxGrid, _F, ctypes.POINTER(_I32), ctypes.POINTER(_I32)],
+    "srfx_tor_scatter_rule": [_I64, SrfxGrid, SrfxTorModel, _U32, ctypes.POINTER(_I32)],
     "srfx_siddon_project": [_P, _I64, _I64, _P, SrfxGrid, _F, _F, _P, _U32, _P],
     "srfx_siddon_backproject": [_P, _I64, _I64, _P, SrfxGrid, _F, _F, _P, _U32, _P],
     "srfx_siddon_backproject_adjoint": [_P, _I64, _I64, _P, SrfxGrid, _F, _F, _P, _U32, _P],
     "srfx_siddon_maplors": [_P, _I64, _I64, _P, SrfxGrid, _P, _U32, _P],
     "srfx_siddon_osem_subset": [_P, _I64, _I64, _P, SrfxGrid, _F, _F, _P, _U32, _P],
     "srfx_siddon_count_nnz": [_P, _I64, _I64, SrfxGrid, _F, _F, _P, _P, _P],
+    "srfx_siddon_scatter_rule": [_I64, SrfxGrid, _F, _F, ctypes.POINTER(_I32)],
     "srfx_mlem_update": [_P, _P, _P, _I64, _P],
     "srfx_frame_copy": [_P, SrfxGrid, _P, _P],
     "srfx_tor_plan_create": [_P, _I64, _I64, _I32, SrfxGrid, SrfxTorModel, SrfxTile,
@@ -223,6 +225,23 @@ def make_tor_model(kernel_width, geo_sigma2_flag, tof_bin, tof_sigma2):
     m.tof_bin = float(tof_bin)
     m.tof_sigma2 = float(tof_sigma2)
     return m
+
+
+def tor_scatter_binned(n, grid, size, model, schedule=None):
+    """Whether an untiled scatter of n events runs binned (model: make_tor_model).
+    Host only."""
+    b = _I32()
+    call("srfx_tor_scatter_rule", int(n), make_grid(grid, (0, 0, 0), size), model,
+         schedule_flags(schedule), ctypes.byref(b))
+    return bool(b.value)
+
+
+def siddon_scatter_binned(n, grid, size, tof_bin, tof_sigma2):
+    """Whether an untiled Siddon scatter of n rays runs binned.  Host only."""
+    b = _I32()
+    call("srfx_siddon_scatter_rule", int(n), make_grid(grid, (0, 0, 0), size), float(tof_bin),
+         float(tof_sigma2), ctypes.byref(b))
+    return bool(b.value)
 
 
 def tor_patch_info(grid, size, kernel_width):

@@ -6,7 +6,9 @@
 
 namespace srfx {
 
-// Whether an untiled scatter of p.n events on stream st runs binned.
+// Whether an untiled scatter of p.n events runs binned by its size and flags, and
+// whether it may on stream st.
+bool binned_rule(const TorParams &p, uint32_t flags);
 bool binned_ok(const TorParams &p, uint32_t flags, hipStream_t st);
 
 // The untiled scatters kBack, kMap, kAdj (p.val, p.out, output strides set)

@@ -241,30 +241,40 @@ int launch_bin_box(const TorParams &p, const TileGeom &g, const BinTables &b, in
 // and 0.137 without TOF: 2.1e6 to 2.4e6 weights by the estimate below.  Beyond,
 // 1M events take 14.0 against 0.98 ms, 1.95 against 0.56, and 55 against 2.4.
 constexpr double kBinnedWeights = 2.4e6;
+// And weights per event: the passes take 0.3 ns and more an event, the time of six
+// direct weights.  Tubes thinner than the voxels have few: 800k events a group,
+// direct and binned us of two groups, 64 x 64 x 32 (6.3 mm, 3 mm tube, 530 ps; 5.7 an
+// event) 541 and 840, 40 x 40 x 20 (10 mm, 4 mm tube; 5.0) 582 and 829, (3 mm, 530 ps;
+// 1.4) 234 and 712; 64 x 64 x 32 (4 mm, 530 ps; 10.2) 900 and 887, 80 x 80 x 40 (5 mm,
+// 3 mm, 530 ps; 11.5) 944 and 935, 40 x 40 x 20 (6 mm; 11.4) 1043 and 874.
+constexpr double kBinnedPerEvent = 10.0;
 
-// Weights of p's events: the tube's cross-section in voxels times the slices
-// of an event, those of the frame or, with TOF, of the +-3 sigma its end points
-// are cut to.
-static double scatter_weights(const TorParams &p, double tof_sigma)
+// Weights of an event: the tube's cross-section in voxels times its slices, those
+// of the frame or, with TOF, of the +-3 sigma its end points are cut to.
+static double event_weights(const TorParams &p)
 {
     const double area = 9.0 * M_PI * p.tor_sigma2 * p.rinter_x * p.rinter_y;
-    const double cut = p.use_tof ? 6.0 * tof_sigma * p.rinter_z : (double)p.gz;
-    return (double)p.n * std::max(1.0, area) * std::min(cut, (double)p.gz);
+    const double cut =
+        p.use_tof ? 6.0 / std::sqrt((double)p.tse_inv) * p.rinter_z : (double)p.gz;
+    return area * std::min(cut, (double)p.gz);
 }
 
-bool binned_ok(const TorParams &p, uint32_t flags, hipStream_t st)
+bool binned_rule(const TorParams &p, uint32_t flags)
 {
     // a schedule in the flags asks for the direct kernels
     constexpr uint32_t sched = (3u << SRFX_LPE_SHIFT) | (3u << SRFX_BLOCK_SHIFT) |
                                (3u << SRFX_SLAB_SHIFT) | SRFX_FULL_PATCH;
-    const double tof_sigma = p.use_tof ? 1.0 / std::sqrt((double)p.tse_inv) : 0.0;
-    if ((flags & sched) || scatter_weights(p, tof_sigma) < kBinnedWeights)
+    const double w = event_weights(p);
+    if ((flags & sched) || w < kBinnedPerEvent || w * (double)p.n < kBinnedWeights)
         return false;
     // the tables of the plan passes index tiles with 24 bits
     const TileGeom g = bin_geom(p);
-    if ((int64_t)g.nwx * g.nwy * g.nslab >= (1 << 20))
-        return false;
-    return workspace_ok(st);
+    return (int64_t)g.nwx * g.nwy * g.nslab < (1 << 20);
+}
+
+bool binned_ok(const TorParams &p, uint32_t flags, hipStream_t st)
+{
+    return binned_rule(p, flags) && workspace_ok(st);
 }
 
 int binned_scatter(int mode, const TorParams &p, hipStream_t st, bool *done)

@@ -240,3 +240,17 @@ extern "C" int srfx_siddon_count_nnz(const float *lors, int64_t n, int64_t ld, s
                        (hipStream_t)stream, p);
     return launch_status();
 }
+
+extern "C" int srfx_siddon_scatter_rule(int64_t n, srfx_grid grid, float tof_bin,
+                                        float tof_sigma2, int32_t *binned)
+{
+    SidParams p;
+    if (n < 0 || !binned)
+        return SRFX_EINVAL;
+    const int rc = siddon_setup(p, nullptr, 0, 0, grid, tof_bin, tof_sigma2);
+    if (rc)
+        return rc;
+    p.n = n;
+    *binned = siddon_binned_rule(p) ? 1 : 0;
+    return SRFX_OK;
+}

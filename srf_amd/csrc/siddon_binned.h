@@ -9,7 +9,9 @@ namespace srfx {
 int siddon_setup(SidParams &p, const float *lors, int64_t n, int64_t ld, const srfx_grid &g,
                  float tof_bin, float tof_sigma2);
 
-// Whether an untiled scatter of p.n rays on stream st runs binned.
+// Whether an untiled scatter of p.n rays runs binned by its size, and whether it
+// may on stream st.
+bool siddon_binned_rule(const SidParams &p);
 bool siddon_binned_ok(const SidParams &p, hipStream_t st);
 
 // The untiled scatters kBack, kMap, kAdj (p.val, p.out set) and the OSEM pass

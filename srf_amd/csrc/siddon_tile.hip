@@ -930,7 +930,7 @@ constexpr double kBinnedWeights = 2.0e6;
 
 namespace srfx {
 
-bool siddon_binned_ok(const SidParams &p, hipStream_t st)
+bool siddon_binned_rule(const SidParams &p)
 {
     for (int c = 0; c < 3; c++)
         if (p.g[c] >= 65536)
@@ -947,7 +947,12 @@ bool siddon_binned_ok(const SidParams &p, hipStream_t st)
     if (planes * (double)p.n < kBinnedWeights)
         return false;
     const SidTileGeom g = tile_geom(p, {16, 16, 8});
-    return (int64_t)g.nt[0] * g.nt[1] * g.nt[2] < (1 << 20) && workspace_ok(st);
+    return (int64_t)g.nt[0] * g.nt[1] * g.nt[2] < (1 << 20);
+}
+
+bool siddon_binned_ok(const SidParams &p, hipStream_t st)
+{
+    return siddon_binned_rule(p) && workspace_ok(st);
 }
 
 int siddon_binned_scatter(int mode, const SidParams &p, hipStream_t st, bool *done)

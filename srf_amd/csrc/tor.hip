@@ -268,3 +268,19 @@ extern "C" int srfx_tor_patch_info(srfx_grid grid, float kernel_width, int32_t *
         *box = p.box;
     return SRFX_OK;
 }
+
+extern "C" int srfx_tor_scatter_rule(int64_t n, srfx_grid grid, srfx_tor_model model,
+                                     uint32_t flags, int32_t *binned)
+{
+    TorParams p;
+    const float one = 1.0f;
+    if (n < 0 || !binned)
+        return SRFX_EINVAL;
+    const int rc = setup(p, &one, 0, 0, grid, model.kernel_width, model.geo_sigma2_flag,
+                         model.tof_bin, model.tof_sigma2);
+    if (rc)
+        return rc;
+    p.n = n;
+    *binned = binned_rule(p, flags) ? 1 : 0;
+    return SRFX_OK;
+}
