@@ -14,13 +14,13 @@
 //   bin_scan            slots and chunks of the tiles (one workgroup);
 //   plan_set_pass<1>    the listings with their slices;
 //   bin_sort            listings of a chunk ordered by length;
-//   record_proj_kernel  (OSEM pass) projections into the records;
+//   bin_project         (OSEM pass) projections into the records;
 //   bin_scatter         workgroups pull chunks: LDS tile, flush.
 // The listing array is sized for the longest average an event set of one axis
 // group can have (every event across the whole frame at 45 degrees along both
 // in-slice axes).  An event set beyond that (events far from the slice axis)
-// leaves the tables empty and sets a flag on which bin_direct, the direct
-// scatter, runs instead of returning at once.
+// leaves the chunk table empty and sets a flag on which the passes after the scan
+// return at once and bin_direct, the direct scatter, runs.
 #include <algorithm>
 
 #include "binned.h"
@@ -105,9 +105,6 @@ __global__ __launch_bounds__(kScanThreads) void bin_scan(BinTables b, TileGeom g
         b.state->over = over;
         b.state->nchunks = over ? 0 : nch;
     }
-    if (over) // the fill pass then writes no slot
-        for (int t = threadIdx.x; t < nt; t += kScanThreads)
-            b.cnt[t] = 0;
 }
 
 __global__ __launch_bounds__(256) void bin_sort(BinTables b)
@@ -135,6 +132,18 @@ __global__ __launch_bounds__(256, NB == 4 ? (ONE ? 4 : 3) : (ONE ? 5 : 4)) void 
             break;
         scatter_chunk<MODE, NB, VREC, ONE, false>(p, g, b.chunks[c], b.list0, b.rec0, ldsd);
     }
+}
+
+// record_proj_kernel<NB, 4, FRAME> of a set that fits.
+template <int NB, bool FRAME>
+__global__ __launch_bounds__(256, NB == 3 && FRAME ? 5 : 4) void bin_project(
+    TorParams p, float4 *rec, const BinState *state)
+{
+    if (state->over)
+        return;
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t e = gid / 64 * 16 + (int)(gid % 16);
+    record_project<NB, 4, FRAME>(p, rec, e, (int)(gid % 64) / 16, e < p.n);
 }
 
 // The direct scatter, for an event set that did not fit.
@@ -202,11 +211,11 @@ int launch_bin(const TorParams &p, const TileGeom &g, const BinTables &b, int cu
         q.img_bytes = (int)bytes;
         if (p.sx == 1 && p.sy == p.gx && p.sz == p.gx * p.gy && bytes < ((int64_t)1 << 31) &&
             (int64_t)p.gx * p.gy < ((int64_t)1 << 24))
-            hipLaunchKernelGGL((record_proj_kernel<NB, 4, true>), dim3(blocks_for(4 * p.n, 256)),
-                               dim3(256), 0, st, q, b.rec0, (float *)nullptr);
+            hipLaunchKernelGGL((bin_project<NB, true>), dim3(blocks_for(4 * p.n, 256)), dim3(256),
+                               0, st, q, b.rec0, b.state);
         else
-            hipLaunchKernelGGL((record_proj_kernel<NB, 4, false>), dim3(blocks_for(4 * p.n, 256)),
-                               dim3(256), 0, st, q, b.rec0, (float *)nullptr);
+            hipLaunchKernelGGL((bin_project<NB, false>), dim3(blocks_for(4 * p.n, 256)),
+                               dim3(256), 0, st, q, b.rec0, b.state);
     }
     int rc = launch_bin_scatter<osem ? kBack : MODE, NB, osem>(p, g, b, cus, st);
     if (rc)
@@ -327,6 +336,7 @@ int binned_scatter(int mode, const TorParams &p, hipStream_t st, bool *done)
     a.fill = b.fill;
     a.off = b.off;
     a.err = &b.state->err;
+    a.skip = &b.state->over;
     a.other = &b.state->other;
     int rc = SRFX_OK;
     for (int64_t e0 = 0; e0 < p.n && !rc; e0 += piece) {

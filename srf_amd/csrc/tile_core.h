@@ -395,6 +395,7 @@ struct PlanSetArgs {
     int *fill;              // fill pass: slots taken per (plan, tile)
     int *const *list;       // fill pass: [nplans] list entries
     int *err;               // fill pass: listings that did not fit
+    const int *skip;        // fill pass: nothing to do where set (nullable)
     int *other;             // count pass: per plan, set to 1 if an event needs
                             // another walk than the NB x (NB - 1) box
 };
@@ -480,6 +481,8 @@ __global__ __launch_bounds__(256) void plan_set_pass(TorParams p, TileGeom g, Pl
     // LDS: with queues, [FillEvent x 256][4 queues of a.queue entries][4
     // queue lengths] first; then [counts (FILL: + bases, ranks)][ntiles]
     extern __shared__ int4 sh4[];
+    if (FILL && a.skip && *a.skip)
+        return;
     const bool queued = FILL && a.queue > 0;
     const int qcap = a.queue;
     char *const shb = reinterpret_cast<char *>(sh4);

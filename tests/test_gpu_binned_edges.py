@@ -123,3 +123,27 @@ def test_siddon_pieces(n, ts2):
                 parts(lambda l, s: ops.siddon_maplors(X, *geo, l, V[s]))) <= 1e-5
     assert _rel(ops.siddon_osem_subset(L, X, *geo, 6.0, ts2),
                 parts(lambda l, s: ops.siddon_osem_subset(l, X, *geo, 6.0, ts2))) <= 1e-5
+
+
+@pytest.mark.parametrize("kw", [4.0, 5.0, 8.0])
+def test_sets_that_do_not_fit(kw):
+    """Lines far from the slice axis list more tiles than the array holds: every pass
+    after the count returns and the direct scatter runs, also in the OSEM pass."""
+    grid, size, n = (200, 60, 24), (400.0, 120.0, 48.0), 60_000
+    r = np.random.default_rng(5)
+    mid = r.uniform(-0.9, 0.9, (n, 3)) * np.asarray(size) / 2
+    d = np.column_stack([40.0 * r.choice([-1, 1], n), r.uniform(-1, 1, n), np.ones(n)])
+    t = r.uniform(0.5, 1.0, n)[:, None] * size[2]
+    p1, p2 = mid - d * t, mid + d * t
+    pc = p1 + r.uniform(0.3, 0.7, n)[:, None] * (p2 - p1)
+    lors = torch.from_numpy(np.ascontiguousarray(
+        np.vstack([p1.T, p2.T, pc.T, np.ones((1, n))]), np.float32)).to(DEV)
+    v = torch.rand(n, device=DEV) + 0.5
+    x = torch.rand(grid[::-1], device=DEV) + 0.5
+    args = (grid, (0.0, 0.0, 0.0), size)
+    assert _lib.tor_scatter_binned(n, grid, size, _lib.make_tor_model(kw, False, *NO_TOF))
+    direct = dict(schedule=(1, 256))
+    b = ops.backprojection(x, lors, v, *args, *NO_TOF, kw, False)
+    assert _rel(b, ops.backprojection(x, lors, v, *args, *NO_TOF, kw, False, **direct)) <= 1e-5
+    b = ops.osem_subset(lors, x, *args, kw, False, *NO_TOF)
+    assert _rel(b, ops.osem_subset(lors, x, *args, kw, False, *NO_TOF, **direct)) <= 1e-5
