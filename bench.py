@@ -22,6 +22,7 @@ each group's kernels launched alone); cpu_baseline = the FP32 CPU
 port of the reference kernels on a bounded sample of the same events.
 """
 import argparse
+import gc
 import json
 import os
 import sys
@@ -304,6 +305,10 @@ def main():
 
     for _ in range(args.warmup):
         osem.iterate(image, 1)
+    # a full garbage collection of the imported modules takes the host 40 ms, three
+    # iterations; when one is due depends on what ran before (compiling the .pyc files
+    # of a first run is enough), so it runs here
+    gc.collect()
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     s0, s1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
