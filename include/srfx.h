@@ -66,12 +66,12 @@ enum srfx_status {
  * Without any schedule flag a large scatter (backprojection, adjoint, Maplors,
  * OSEM pass; ~2.4e6 weights and up, ten an event and up; srfx_tor_scatter_rule)
  * runs binned: its events are listed by image tile on the device and every tile
- * accumulated in LDS, with a stream-ordered
- * workspace of up to 256 MiB from the device's memory pool (a stream under
- * capture, or a failed allocation, keeps the kernels without workspace).
+ * accumulated in LDS, with a stream-ordered workspace of up to 256 MiB (a stream
+ * under capture, or a failed allocation, keeps the kernels without workspace).
  * Likewise the projection of more than 131072 events over an image of 10 MB
  * and up walks the events in a locality order formed on the device (up to 156
- * MiB of workspace). */
+ * MiB of workspace).  Workspaces come from a memory pool of the library's own, one
+ * a device, which keeps up to 1 GiB between calls (srfx_workspace_trim). */
 #define SRFX_LPE_SHIFT 4
 #define SRFX_LPE_1 (1u << SRFX_LPE_SHIFT)
 #define SRFX_LPE_4 (2u << SRFX_LPE_SHIFT)
@@ -87,7 +87,7 @@ enum srfx_status {
  * chip's 8 XCDs gathers from and scatters into one eighth of the image;
  * SRFX_SLAB_BLOCKED8 is the same work without that affinity; SRFX_SLAB_XCD16
  * uses 16 slabs, two per XCD.  Projection and OSEM then take a stream-ordered
- * workspace of (slabs x n) floats from the device's memory pool.  Lanes per
+ * workspace of (slabs x n) floats.  Lanes per
  * event is 1 under a slab schedule. */
 #define SRFX_SLAB_SHIFT 8
 #define SRFX_SLAB_XCD8 (1u << SRFX_SLAB_SHIFT)
@@ -180,7 +180,7 @@ int srfx_tor_count_nnz(const float *lors, int64_t n, int64_t ld, srfx_grid grid,
  * SRFX_SLAB_* field, SRFX_SLAB_XCD8 when it names none), with the per-slab
  * partial projections in a static scratch of the library (16 MiB per device,
  * 2^22 floats, kept until the process ends) instead of a workspace from the
- * device's memory pool.  Calls no allocating routine.  Limit: slabs x n <=
+ * memory pool.  Calls no allocating routine.  Limit: slabs x n <=
  * 2^22 (n <= 524288 events at 8 slabs, 262144 at 16); larger inputs return
  * SRFX_ETOOLARGE before any device work (split them and pass
  * SRFX_ACCUMULATE).  Every partial is written before it is read, so nothing
@@ -382,7 +382,7 @@ int srfx_split_lors_fill(const void *rows, int64_t n, int64_t row_stride, int64_
  * mm), then by the Morton interleave of the two slopes (slope_bin) and the
  * crossing with the plane z = center_z (pos_bin mm).  soa: [ncols >= 9, n], row
  * stride ld; out (nullable): the reordered [ncols, n].  Stream-ordered
- * workspace from the device's memory pool. */
+ * workspace. */
 int srfx_locality_sort(const float *soa, int64_t n, int64_t ld, int32_t ncols,
                        int32_t nb_subsets, double center_z, double zc_bin, double slope_bin,
                        double pos_bin, float *out, int64_t *order, void *stream);
@@ -518,6 +518,11 @@ int srfx_tor_batch_set_schedule(srfx_tor_batch *plan, int32_t lanes_per_event,
 int srfx_tor_batch_destroy(srfx_tor_batch *plan);
 
 /* ------------------------------------------------------------- Update --- */
+
+/* Return the current device's unused workspace memory (the pool beside
+ * SRFX_LPE_SHIFT) to the device.  Workspaces of calls still running stay.  No
+ * reference counterpart. */
+int srfx_workspace_trim(void);
 
 /* mlem_update, model/recon_step.py:48-49: x <- x * emap * bp (elementwise,
  * n voxels, evaluated as (x * emap) * bp). */

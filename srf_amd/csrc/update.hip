@@ -1,6 +1,6 @@
 // Elementwise kernels: output zeroing (a fill kernel, so the ops stay
 // capturable in HIP graphs) and the MLEM image update.
-#include <atomic>
+#include <mutex>
 
 #include "common.h"
 
@@ -72,24 +72,53 @@ int zero_grid(float *img, const srfx_grid &g, uint32_t flags, hipStream_t st)
     return launch_status();
 }
 
+// The workspaces' memory pool of each device: one of its own, so that its release
+// threshold concerns nobody else.  It keeps freed workspaces, up to kKeptBytes
+// (three of the largest calls at once), instead of returning them to the driver
+// at every synchronisation (a call that maps its memory again takes milliseconds);
+// srfx_workspace_trim returns the rest.
+constexpr uint64_t kKeptBytes = 1ull << 30;
+constexpr int kMaxDevices = 64;
+
+static std::mutex pool_mutex;
+static hipMemPool_t pools[kMaxDevices];
+
+// The current device's pool, or null.
+static hipMemPool_t workspace_pool(bool create)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices)
+        return nullptr;
+    std::lock_guard<std::mutex> lock(pool_mutex);
+    if (!pools[dev] && create) {
+        hipMemPoolProps props{};
+        props.allocType = hipMemAllocationTypePinned;
+        props.handleTypes = hipMemHandleTypeNone;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = dev;
+        hipMemPool_t pool = nullptr;
+        uint64_t keep = kKeptBytes;
+        if (hipMemPoolCreate(&pool, &props) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipMemPoolDestroy(pool);
+            return nullptr;
+        }
+        pools[dev] = pool;
+    }
+    return pools[dev];
+}
+
 int ws_alloc(void **ptr, size_t bytes, hipStream_t st)
 {
-    // Keep freed workspace in the pool instead of returning it to the driver
-    // at every synchronisation (once per device).
-    static std::atomic<uint64_t> pool_set{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess)
-        return SRFX_ELAUNCH;
-    uint64_t bit = 1ull << (dev & 63);
-    if (!(pool_set.load() & bit)) {
-        hipMemPool_t pool;
-        if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) {
-            uint64_t thr = UINT64_MAX;
-            (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &thr);
-        }
-        pool_set.fetch_or(bit);
-    }
-    if (hipMallocAsync(ptr, bytes ? bytes : 256, st) != hipSuccess) {
+    bytes = bytes ? bytes : 256;
+    // under capture the allocation is the graph's own
+    const hipMemPool_t pool = workspace_ok(st) ? workspace_pool(true) : nullptr;
+    if ((pool ? hipMallocFromPoolAsync(ptr, bytes, pool, st) : hipMallocAsync(ptr, bytes, st)) !=
+        hipSuccess) {
         (void)hipGetLastError();
         return SRFX_ENOMEM;
     }
@@ -145,4 +174,14 @@ extern "C" const char *srfx_strerror(int status)
     default:
         return "unknown status";
     }
+}
+
+extern "C" int srfx_workspace_trim(void)
+{
+    const hipMemPool_t pool = workspace_pool(false);
+    if (pool && hipMemPoolTrimTo(pool, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return SRFX_ELAUNCH;
+    }
+    return SRFX_OK;
 }

@@ -290,3 +290,9 @@ def mlem_update(x, emap, bp):
         raise ValueError("x, emap and bp must have the same number of voxels")
     _lib.call("srfx_mlem_update", _ptr(x), _ptr(emap), _ptr(bp), x.numel(), _stream())
     return x
+
+
+def release_workspace():
+    """Return the memory that untiled calls keep for their workspaces (up to 1 GiB
+    on the current device) to the device (srfx_workspace_trim)."""
+    _lib.call("srfx_workspace_trim")
