@@ -219,7 +219,8 @@ ZC_BIN, SLOPE_BIN, POS_BIN = 40.0, 0.04, 6.0
 
 def _sortable(soa, nb_subsets):
     return (_native(soa) and soa.dtype == torch.float32 and soa.shape[0] >= 9
-            and soa.shape[1] < 2 ** 31 - 1 and 1 <= nb_subsets <= 1 << 24
+            and soa.shape[1] < 2 ** 31 - 1 and hasattr(nb_subsets, "__index__")
+            and 1 <= nb_subsets <= 1 << 24
             and soa.stride(1) == 1 and soa.stride(0) >= soa.shape[1])
 
 
@@ -244,7 +245,7 @@ def locality_order(soa, nb_subsets, center_z=0.0):
     if _sortable(soa, nb_subsets):
         return _locality_sort(soa, nb_subsets, center_z, False)[1]
     n = soa.shape[1]
-    if n == 0 and soa.shape[0] >= 9:
+    if n == 0 and soa.shape[0] >= 9 and hasattr(nb_subsets, "__index__"):
         return torch.empty(0, dtype=torch.int64, device=soa.device)
     key = locality_key(soa, center_z)
     order = torch.empty(n, dtype=torch.int64, device=soa.device)
