@@ -17,12 +17,13 @@ Row order inside a group is the reference's: ascending event index
 float32 and float64 rows on a GPU go through the HIP kernels
 (srfx_split_lors_*, srfx_locality_sort), which give the same bits; other rows
 (host tensors, other types, rows that carry a gradient or a tangent, calls under
-stream capture) through the torch operations below.
+a tracer, a dispatch mode or stream capture) through the torch operations below.
 """
 import ctypes
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._python_dispatch import is_in_torch_dispatch_mode
 
 from . import _lib
 
@@ -105,6 +106,7 @@ def _native(t):
     return (type(t) is torch.Tensor and t.device.type == "cuda" and not t.requires_grad
             and t.dim() == 2 and t.numel() > 0 and not t.is_neg()
             and forward_ad.unpack_dual(t).tangent is None
+            and not torch.jit.is_tracing() and not is_in_torch_dispatch_mode()
             and not torch.cuda.is_current_stream_capturing())
 
 
