@@ -195,7 +195,7 @@ int srfx_tor_osem_subset_noalloc(const float *lors, int64_t n, int64_t ld, const
  * the candidate box the kernels compile for it: 3 or 4 (NB x NB voxels per
  * slice hold every kept voxel of an event whose slice axis is its dominant
  * direction), or 0 when the ellipse of such an event can span more than 4
- * voxels (the generic chord walk).  Host only: no device work.  Either
+ * voxels (the row and chord walks).  Host only: no device work.  Either
  * output pointer may be NULL.  SRFX_EUNSUPPORTED for P > 16, as the ops. */
 int srfx_tor_patch_info(srfx_grid grid, float kernel_width, int32_t *patch, int32_t *box);
 
@@ -314,7 +314,7 @@ int srfx_tor_plan_create_subset_groups(const srfx_subset_group *groups, int32_t 
 /* Listings (event, tile pairs) and workgroup chunks of a plan. */
 int srfx_tor_plan_info(srfx_tor_plan plan, int64_t *nlistings, int32_t *nchunks);
 
-/* The candidate box of the plan's walks (3 or 4; 0: chord walks) and
+/* The candidate box of the plan's walks (3 or 4; 0: row walks) and
  * whether every event walks the NB x (NB - 1) box.  With box 3, such a plan
  * scatters through the kernel that holds only that walk when its tile takes
  * at most a fifth of a CU's LDS.  No reference counterpart. */

@@ -248,7 +248,7 @@ def siddon_scatter_binned(n, grid, size, tof_bin, tof_sigma2):
 def tor_patch_info(grid, size, kernel_width):
     """(P, box) for a TOR op frame (grid (gx, gy, gz), full size in mm): the
     reference's patch width P (tor.cu.cc:375) and the candidate box the
-    kernels run (3, 4, or 0 for the generic chord walk).  Host only."""
+    kernels run (3, 4, or 0 for wider tubes: row and chord walks).  Host only."""
     p, b = _I32(), _I32()
     call("srfx_tor_patch_info", make_grid(grid, (0, 0, 0), size), float(kernel_width),
          ctypes.byref(p), ctypes.byref(b))

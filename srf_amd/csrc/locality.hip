@@ -211,8 +211,8 @@ __global__ __launch_bounds__(256) void locality_count(TorParams p, int64_t K, in
 }
 
 // Exclusive prefix sums of the counts: workgroup b scans kScan counts and adds
-// the sum of all before them, which it reads itself (64 workgroups at most, the
-// counts stay in L2).
+// the sum of all before them, which it reads itself (64 workgroups unless the
+// subsets alone take more buckets than 2^16; the counts stay in L2).
 __global__ __launch_bounds__(kScan) void locality_scan(const unsigned *__restrict__ hist,
                                                        unsigned *__restrict__ first, int64_t n)
 {

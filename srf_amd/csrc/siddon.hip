@@ -3,8 +3,10 @@
 // siddon_core.h.
 //
 // Unlike the reference, a ray whose start voxel falls outside the grid is
-// skipped (the reference indexes out of bounds there), and the walk is capped
-// at gx+gy+gz+3 steps; both only affect degenerate rays.
+// skipped (the reference indexes out of bounds there), and walks are bounded: the
+// count by gx+gy+gz+3 steps, the others by the crossing that leaves the image, at
+// most one slab for each plane of the dominant axis; both only affect degenerate
+// rays.
 #include "siddon_binned.h"
 
 namespace srfx {

@@ -3,13 +3,15 @@
 //
 // Semantics follow the reference CUDA op src/cpp/tf_custom_ops/siddon.cu.cc
 // (CreateRay 61-81, ClipRay / IsThroughImage 118-183, SetupRayCast 196-284,
-// RayTracing / BackRayTracing / Map 293-415).  Ray geometry and traversal
-// (clip, start voxel, nextT updates, argmin, segment lengths and the TOF
-// distance) are carried in FP64 with explicitly rounded operations in the
-// reference's source order, so the visited voxels are those of the FP64
-// restatement, including rays lying exactly on voxel faces, whose voxel is
-// otherwise decided by FP32 rounding.  Weights (1/L^2, the TOF Gaussian) and
-// the accumulation are FP32.
+// RayTracing / BackRayTracing / Map 293-415).  Ray geometry (clip, start voxel,
+// first crossings) is formed in FP64 with explicitly rounded operations in the
+// reference's source order, so a ray enters through the voxel of the FP64
+// restatement, also where it lies exactly on a voxel face.  The count follows the
+// reference's traversal step by step (nextT updates, argmin); the other walks form
+// crossing k of an axis as n + k t (spans, below), whose segments are the
+// traversal's up to the rounding of that product.  Segment lengths, TOF distance and
+// variance are FP64; weights (1/L^2, the TOF Gaussian) and the accumulation are
+// FP32.
 #pragma once
 
 #include <float.h>

@@ -22,7 +22,7 @@
 //            each event's partials in the event's own listing order, so the
 //            projection is deterministic.
 // The voxels an event visits and their weights are those of the untiled
-// kernels (tor_core.h): the tile walk is the candidate-box (or chord) walk
+// kernels (tor_core.h): the tile walk is the candidate-box, row or chord walk
 // clipped to the window.
 #pragma once
 
@@ -159,10 +159,6 @@ __host__ __device__ inline bool flush_y_fastest(const TorParams &p)
 {
     return (p.oy < 0 ? -p.oy : p.oy) < (p.ox < 0 ? -p.ox : p.ox);
 }
-
-// Index of voxel (ix, iy) of slice s in the LDS tile of box b: x fastest, or
-// (YF) y fastest, so that a flush along the tile's fastest axis writes
-// consecutive addresses of an output whose unit stride is along op y.
 
 // Narrow [s0, s1] to the slices s with lo <= u(s) <= hi, u(s) = a + s b,
 // rb = 1 / b (FP64; the bounds on s are widened by 1e-6 slice, so the result
@@ -654,6 +650,9 @@ __global__ __launch_bounds__(256) void fill_int(int *v, int64_t n, int value)
         v[i] = value;
 }
 
+// Index of voxel (ix, iy) of slice s in the LDS tile of box b: x fastest, or
+// (YF) y fastest, so that a flush along the tile's fastest axis writes
+// consecutive addresses of an output whose unit stride is along op y.
 template <bool YF>
 __device__ __forceinline__ int lds_index(const TileGeom &g, const TileBox &b, int s, int ix, int iy)
 {
@@ -667,8 +666,7 @@ __device__ __forceinline__ int lds_index(const TileGeom &g, const TileBox &b, in
 template <int KIND, bool YF, typename T>
 __device__ __forceinline__ float window_walk(const TorParams &p, const TileGeom &g,
                                              const TileBox &b, const Event &ev, const Track &t,
-                                             const Cross &c, float amp, int s, float scale,
-                                             T *lds)
+                                             const Cross &c, float amp, int s, T *lds)
 {
     const int P = p.patch;
     int i_lo = max(0, b.x0 - c.ix0), i_hi = min(P - 1, b.x1 - c.ix0);
@@ -903,7 +901,7 @@ __device__ __forceinline__ void scatter_chords(const TorParams &p, const TileGeo
         Cross c;
         cross_at(p, ev, t, ax, s, c);
         const float amp = tof ? tof_exp(p, ev, t, s) * ts : scale;
-        window_walk<1, true>(p, g, b, ev, t, c, amp, s, scale, lds);
+        window_walk<1, true>(p, g, b, ev, t, c, amp, s, lds);
     }
 }
 
@@ -937,7 +935,7 @@ __device__ __forceinline__ float gather_event(const TorParams &p, const TileGeom
                 acc += slice_box<0, NBB, NBB, true>(p, ev, t, c, amp, s, il, ih, jl, jh, idx,
                                                     lds, lds);
         } else {
-            acc += window_walk<0, false>(p, g, b, ev, t, c, amp, s, 0.0f, lds);
+            acc += window_walk<0, false>(p, g, b, ev, t, c, amp, s, lds);
         }
     }
     return acc;

@@ -59,7 +59,7 @@ struct TorParams {
     float finter_x, finter_y;
     float rfinter_x, rfinter_y;
     int patch, half;
-    int box;        // compiled candidate box (3, 4) or 0 (chord walk only)
+    int box;        // compiled candidate box (3, 4) or 0 (wider tubes: row and chord walks)
     int full_patch; // evaluate every patch voxel (reference loop) instead of the chords
     int geo;
     int use_tof;
@@ -1124,7 +1124,8 @@ __device__ __forceinline__ float slice_rows_frame(const TorParams &p, const Even
 
 // Box shape of an event for a compiled box size NB: 1 = NB x (NB - 1)
 // (enough for every event whose ellipse spans at most NB - 1 rows, e.g. all
-// C2 events), 2 = NB x NB, 0 = larger (chord walk).
+// C2 events), 2 = NB x NB, 0 = larger (chord walk; NB = 0: the row walk where the
+// image is an op frame or a plan's tile).
 template <int NB>
 __device__ __forceinline__ int box_shape(const Track &t)
 {
@@ -1430,7 +1431,8 @@ int setup(TorParams &p, const float *lors, int64_t n, int64_t ld, const srfx_gri
     // Candidate box: the compiled size that holds the box of every event
     // whose slice axis is its dominant direction (as in the axis groups of
     // on_tor_lors.py): there the ellipse's half extents are at most
-    // sqrt(2 tm).  Events with a larger box take the chord walk.
+    // sqrt(2 tm).  Single events with a larger box take the chord walk; tubes
+    // wider than every compiled box (0) the row walk from op frames and in tiles.
     {
         double tm = 9.0 * p.tor_sigma2 * (1.0 + 1.0e-5) + 2.0 * kThrMargin;
         double h = std::sqrt(2.0 * tm);

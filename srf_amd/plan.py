@@ -166,7 +166,7 @@ class TorPlan:
         return int(a.value), int(b.value)
 
     def walks(self):
-        """(candidate box 3 or 4, or 0 for chord walks; whether every event
+        """(candidate box 3 or 4, or 0 for row walks; whether every event
         walks the NB x (NB - 1) box, so that the scatter can run its
         single-walk kernel)."""
         a, b = ctypes.c_int32(), ctypes.c_int32()
