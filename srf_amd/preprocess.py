@@ -104,9 +104,9 @@ def _as64(lors, ncols):
 
 def _native(t):
     return (type(t) is torch.Tensor and t.device.type == "cuda" and not t.requires_grad
+            and not torch.jit.is_tracing() and not is_in_torch_dispatch_mode()
             and t.dim() == 2 and t.numel() > 0 and not t.is_neg()
             and forward_ad.unpack_dual(t).tangent is None
-            and not torch.jit.is_tracing() and not is_in_torch_dispatch_mode()
             and not torch.cuda.is_current_stream_capturing())
 
 
