@@ -405,7 +405,7 @@ int srfx_tor_plan_osem_groups(const srfx_tor_plan *plans, int32_t nplans, const 
  * the same LORs, with the same voxels and segment values, summed in another
  * order).  A plan lists each LOR in the image tiles of tx x ty x tz voxels it
  * crosses (tx * ty * tz <= 8192: the scatter's tile is FP64 in LDS); a scatter
- * workgroup takes up to `chunk` listings of one tile (0: 256 to 2048 by the
+ * workgroup takes up to `chunk` listings of one tile (0: 1024 to 2048 by the
  * plan's listings), accumulates them in LDS and flushes the tile with one
  * atomic per non-zero voxel.  `block`: 64, 128 or 256
  * (0 = 256).  `sort` nonzero: the plan keeps a copy of its LORs sorted by

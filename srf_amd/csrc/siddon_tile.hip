@@ -45,15 +45,20 @@ constexpr int kRayBits = 27;
 
 // Listings per workgroup where the caller names no chunk: as few as let every
 // workgroup of the scatter run at once (`slots`), so that a small set fills the
-// chip, and no more than 2048, beyond which the flushes no longer count.
-// Scatter of 20k, 125k and 1M LORs (128 x 128 x 64), chunks of 512, 1024 and
-// 2048: 26, 29 and 36 us; 75, 57 and 69; 538, 338 and 286.
-constexpr int kChunkMin = 256, kChunkMax = 2048;
+// chip, and no more than 2048, beyond which the flushes no longer count; no fewer
+// than `least`.  A binned call's least is 256: its sums are FP64 until one flush a
+// chunk, and projection and backprojection of 100k LORs (128 x 128 x 64) take 204
+// us, 220 with 1024.  A plan's least is 1024: every flush adds an FP32 rounding to
+// the image, and an OSEM pass of 500k LORs (same image, four subsets) is
+// 1.235e-7 from 64 bits with it, 1.313e-7 with 2048 alone and 1.338e-7 with 256;
+// 519, 632 and 530 us.  A pass of 30k, 80k and 160k LORs takes 153, 213 and 324 us
+// with 256 and 169, 225 and 285 with 1024.
+constexpr int kChunkMin = 256, kPlanChunkMin = 1024, kChunkMax = 2048;
 
-__host__ __device__ inline int auto_chunk(long long listings, int slots)
+__host__ __device__ inline int auto_chunk(long long listings, int slots, int least)
 {
     const long long c = (listings / slots + kChunkMin - 1) / kChunkMin * kChunkMin;
-    return (int)(c < kChunkMin ? kChunkMin : (c > kChunkMax ? kChunkMax : c));
+    return (int)(c < least ? least : (c > kChunkMax ? kChunkMax : c));
 }
 
 struct SidTileGeom {
@@ -456,7 +461,7 @@ __global__ __launch_bounds__(kScanThreads) void sid_bin_scan(SidBins b, int nt, 
         sum += (long long)b.cnt[q];
     long long listings;
     (void)block_scan<kScanThreads>(sum, listings);
-    const int chunk = auto_chunk(listings, slots);
+    const int chunk = auto_chunk(listings, slots, kChunkMin);
     for (int q0 = 0; q0 < nt; q0 += kScanThreads) {
         const int q = q0 + (int)threadIdx.x;
         const int c = q < nt ? (int)b.cnt[q] : 0;
@@ -852,7 +857,8 @@ int build_set(const float *lors, int64_t n, int64_t ld, const srfx_grid &grid, f
         unsigned long long listings = 0;
         for (int tt = 0; tt < ntiles; tt++)
             listings += hc[(size_t)k * ntiles + tt];
-        const int chunk = tile.chunk ? tile.chunk : auto_chunk((long long)listings, slots);
+        const int chunk =
+            tile.chunk ? tile.chunk : auto_chunk((long long)listings, slots, kPlanChunkMin);
         max_chunk = std::max(max_chunk, chunk);
         for (int tt = 0; tt < ntiles; tt++) {
             const unsigned long long c = hc[(size_t)k * ntiles + tt];
